@@ -508,6 +508,26 @@ int mk_restrict_tent_f32(const float *x, int32_t B, int32_t H, int32_t W,
                          int32_t f, float *y, void *stream);
 int mk_prolong_tent_f32(const float *y, int32_t B, int32_t H, int32_t W,
                         int32_t f, float *x, int32_t accumulate, void *stream);
+/* M r of a level network outside training, with no channel buffers:
+ * z = s (exp(log_alpha[0]) u + sum_l (R^l)^T C_l^T C_l R^l u), u = s r, on
+ * B x H x W maps.  C_l is level l's 1 -> 16 layer and R^l restricts through
+ * the steps steps[1..l] (host array, each 1..64; steps[0] is not read), by
+ * box (tent == 0) or tent weights.  stencils holds C_l^T C_l as 5x5 stencils
+ * (mk_level_stencils_f32 from the nlevel x 16 x 9 weights, into
+ * mk_level_stencils_floats(nlevel) floats), composed in FP64 and rounded
+ * once; pixels on the image's edge have their own, as the layers' channels
+ * are zero outside it.  z may not overlap r or s.  work:
+ * mk_precon_levels_workspace_bytes bytes (-1 on bad arguments). */
+int64_t mk_level_stencils_floats(int32_t nlevel);
+int mk_level_stencils_f32(const float *w, int32_t nlevel, float *st,
+                          void *stream);
+int64_t mk_precon_levels_workspace_bytes(int32_t nlevel, const int32_t *steps,
+                                         int32_t B, int32_t H, int32_t W);
+int mk_precon_levels_f32(float *z, const float *s, const float *r,
+                         const float *log_alpha, const float *stencils,
+                         int32_t tent, int32_t nlevel, const int32_t *steps,
+                         int32_t B, int32_t H, int32_t W, void *work,
+                         int64_t work_bytes, void *stream);
 /* z = s * (exp(log_alpha[0]) * u + g); g may be NULL (Jacobi-like). */
 int mk_precon_finish_f32(float *z, const float *s, const float *log_alpha,
                          const float *u, const float *g, int64_t n,

@@ -20,8 +20,11 @@ tent    as levels with full-weighting restriction (tent weights) in place of
         and coarse corrections come back smooth.
 
 Every operation is a libmkgpu call (mk_conv3x3_f32, mk_conv3x3_wgrad_f32,
-mk_conv3x3_adjoint_weights, mk_restrict_{box,tent}_f32, mk_prolong_{box,tent}_f32).
+mk_conv3x3_adjoint_weights, mk_restrict_{box,tent}_f32, mk_prolong_{box,tent}_f32;
+mk_precon_levels_f32 for a level network outside training).
 """
+import ctypes
+
 import numpy as np
 import torch
 
@@ -173,16 +176,36 @@ class LevelsNet(_Base):
             h, w = self.dims[-1]
             self.dims.append(((h + st - 1) // st, (w + st - 1) // st))
         B = self.B
-        self.u = [None] + [self._f32(B, 1, h, w) for h, w in self.dims[1:]]  # u[0] is the caller's
-        self.c = [self._f32(B, CH, h, w) for h, w in self.dims]
-        self.gl = [None] + [self._f32(B, 1, h, w) for h, w in self.dims[1:]]  # g[0] is the caller's
         self.train = train
         if train:
+            self.u = [None] + [self._f32(B, 1, h, w) for h, w in self.dims[1:]]  # u[0] is the caller's
+            self.c = [self._f32(B, CH, h, w) for h, w in self.dims]
+            self.gl = [None] + [self._f32(B, 1, h, w) for h, w in self.dims[1:]]  # g[0] is the caller's
             self.ql = [None] + [self._f32(B, 1, h, w) for h, w in self.dims[1:]]
             self.cq = self._f32(B, CH, self.H, self.W)
+        else:  # no activations are kept: C_l^T C_l runs as one composed 5x5 stencil per level
+            self._steps = (ctypes.c_int32 * self.nlayer)(*self.steps)
+            self._tent = int(kind == "tent")
+            nb = int(mkgpu.lib.mk_precon_levels_workspace_bytes(self.nlayer, self._steps, B, self.H, self.W))
+            if nb < 0:
+                raise ValueError("level steps %s or map %d x %d out of range" % (self.steps, self.H, self.W))
+            self.work = self._f32(nb // 4)
+            self.stencils = self._f32(int(mkgpu.lib.mk_level_stencils_floats(self.nlayer)))
 
     def workspace_bytes(self):
         return max(int(mkgpu.lib.mk_conv3x3_wgrad_workspace_bytes(self.B, CH, 1, h, w, 1)) for h, w in self.dims)
+
+    def refresh_adjoint(self):
+        if self.train:
+            return super().refresh_adjoint()
+        mkgpu.check("mk_level_stencils_f32", self.params.data_ptr(), self.nlayer, self.stencils.data_ptr(),
+                    dev.stream_ptr())
+
+    def precondition(self, r, s, z):
+        """z = s (alpha s r + K^T K s r) outside training; z overlaps neither."""
+        mkgpu.check("mk_precon_levels_f32", z.data_ptr(), s.data_ptr(), r.data_ptr(), self.log_alpha_ptr,
+                    self.stencils.data_ptr(), self._tent, self.nlayer, self._steps, self.B, self.H, self.W,
+                    self.work.data_ptr(), self.work.numel() * 4, dev.stream_ptr())
 
     def _restrict(self, x, l, y):
         h, w = self.dims[l - 1]
@@ -194,6 +217,7 @@ class LevelsNet(_Base):
                     dev.stream_ptr())
 
     def forward(self, u, g0):
+        """g0 = K^T K u, keeping the activations (networks built for training)."""
         L = self.nlayer
         us = [u] + self.u[1:]
         gs = [g0] + self.gl[1:]

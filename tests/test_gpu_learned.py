@@ -271,3 +271,40 @@ def test_shipped_weights_gain_over_jacobi(env, fname, arch_want, max_ratio):
     assert lrn["iters"] <= max_ratio * jac["iters"], (lrn["iters"], jac["iters"])
     assert lrn["true_rel_res"] < 3e-6
     assert map_distance(P, lrn["x"], jac["x"]) < 1e-3
+
+
+# Edges of the composed-stencil path: images thinner than the stencil, tiles
+# of 64 x 8 and (from 512 of them) 64 x 32 pixels with remainders, odd and unit
+# steps, a coarse level narrower than its support, and coarse levels inside and
+# outside the one-workgroup tail.  1e-5: a few hundred FP32 roundings of 6e-8
+# at worst.
+@pytest.mark.parametrize("arch,spec,B,H,W", [
+    ("tent", (1,), 1, 1, 1), ("levels", (1, 2), 3, 1, 9), ("tent", (1, 2, 6), 1, 2, 3), ("tent", (1, 1, 4), 1, 7, 64),
+    ("levels", (1, 3, 6, 12), 2, 33, 65), ("tent", (1, 4, 16, 64, 256), 1, 129, 257), ("tent", (1, 64), 1, 130, 200),
+    ("levels", (1, 64, 128), 1, 65, 1000), ("tent", (1, 3), 90, 65, 70), ("levels", (1, 4, 16), 1, 1031, 1025),
+    ("tent", (1, 5, 10, 20), 1, 300, 31)])
+def test_levels_precon_edges(env, arch, spec, B, H, W):
+    torch, device, mkgpu = env
+    from minkasi_amd.learned.nets import make_net
+    p, net, r, _, s, _ = _net_and_data(arch, spec, B, H, W, seed=H + W)
+    s = s + np.float32(0.1)  # no pixel is masked: the smallest images are all corner
+    gnet = make_net(arch, spec, p, B, H, W)
+    gnet.refresh_adjoint()
+    rt, st = _t(env, r), _t(env, s)
+    z = torch.full_like(rt, 3.0)
+    print("levels_precon", arch, spec, B, H, W, flush=True)
+    gnet.precondition(rt, st, z)
+    ref = net.apply(r.astype(np.float64), s.astype(np.float64))
+    assert np.linalg.norm(z.cpu().numpy() - ref) <= 1e-5 * np.linalg.norm(ref)
+
+
+def test_levels_precon_in_place(env):
+    torch, device, mkgpu = env
+    from minkasi_amd.learned.precon import LearnedPrecon
+    p, net, r, _, s, _ = _net_and_data("tent", (1, 4), 1, 41, 66)
+    lp = LearnedPrecon(_t(env, s[0, 0]), p, "tent", (1, 4))
+    rt = _t(env, r[0, 0])
+    z = torch.empty_like(rt)
+    lp.apply_to(rt, z)
+    lp.apply_to(rt, rt)
+    assert torch.equal(rt, z)
