@@ -14,8 +14,9 @@ class _MapsetBase:
 
     def copy(self):
         new_mapset = self.__class__()
-        for i in range(self.nmap):
-            new_mapset.add_map(self.maps[i].copy())
+        for i in range(self.nmap):  # one copy of each member: add_map would copy the copy
+            new_mapset.maps.append(self.maps[i].copy())
+            new_mapset.nmap += 1
         return new_mapset
 
 
