@@ -6,10 +6,8 @@
 //
 //  median_cols   : per sample (column) the median over the detectors (rows),
 //                  numpy semantics (mean of the two middle values for an even
-//                  count).  One wave per column: the column is loaded into
-//                  registers (64 x V values, padded with +inf) and sorted
-//                  with a bitonic network, lanes exchanging through
-//                  __shfl_xor and register pairs swapping in place.
+//                  count), as exact order statistics: one wave per column
+//                  bisects on the values' ordered bit patterns.
 //  design        : X[t][k] = P_k(x_t) (k <= ord) and X[t][ord+1+i] =
 //                  P_i(x_t) cm[t] (i < cm_ord), x_t = (t - (n-1)/2) / ((n-1)/2),
 //                  Legendre P by the three-term recurrence, FP64; also X^T.
@@ -25,64 +23,115 @@ namespace {
 
 constexpr int kWave = 64;
 
+// Bit patterns whose unsigned order is the order of the values.
+__device__ __forceinline__ uint32_t order_key(float v) {
+  const uint32_t u = __float_as_uint(v);
+  return u ^ ((u >> 31) ? 0xffffffffu : 0x80000000u);
+}
+__device__ __forceinline__ uint64_t order_key(double v) {
+  const uint64_t u = (uint64_t)__double_as_longlong(v);
+  return u ^ ((u >> 63) ? ~0ull : 1ull << 63);
+}
+__device__ __forceinline__ float key_value(uint32_t k) {
+  return __uint_as_float(k ^ ((k >> 31) ? 0x80000000u : 0xffffffffu));
+}
+__device__ __forceinline__ double key_value(uint64_t k) {
+  return __longlong_as_double((long long)(k ^ ((k >> 63) ? 1ull << 63 : ~0ull)));
+}
+template <typename T>
+struct KeyOf;
+template <>
+struct KeyOf<float> { using type = uint32_t; };
+template <>
+struct KeyOf<double> { using type = uint64_t; };
+
+// Smallest of the wave, in scalar registers.
+__device__ __forceinline__ uint32_t wave_min(uint32_t v) {
+#pragma unroll
+  for (int d = 32; d; d >>= 1) v = min(v, (uint32_t)__shfl_xor((int)v, d, 64));
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+}
+__device__ __forceinline__ uint64_t wave_min(uint64_t v) {
+#pragma unroll
+  for (int d = 32; d; d >>= 1) v = min(v, (uint64_t)__shfl_xor((unsigned long long)v, d, 64));
+  return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v) |
+         (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32;
+}
+
+// Bound by the scalar work of the bisection.  A workgroup stages C columns
+// through LDS, so rows are read along their length (a wave per column would
+// fetch a line for every value), and a wave then holds a column in V registers
+// a lane.  A step counts the keys up to a pivot with one compare and one
+// population count of the lane mask per register; the bracket starts at the
+// smallest and largest key and closes as soon as one key is left in it, so a
+// column takes about log2(nrow) steps more than its values share leading bits,
+// against (6 + log2 V)(7 + log2 V)/2 exchange stages of a full sort.  215 x
+// 100003 FP32: 65 us from 151 us (bitonic sort over lanes and registers, column
+// loads).
 template <typename T, int V>
 __global__ void __launch_bounds__(256) median_cols_kernel(const T* __restrict__ dat, int64_t nrow, int64_t ncol,
-                                                          int64_t ld, T* __restrict__ out) {
-  const int lane = threadIdx.x & 63;
-  const int64_t c = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (c >= ncol) return;  // whole wave
-  constexpr int N = kWave * V;
-  T x[V];
-#pragma unroll
-  for (int e = 0; e < V; e++) {
-    const int64_t i = (int64_t)e * kWave + lane;
-    x[e] = i < nrow ? dat[i * ld + c] : T(INFINITY);
+                                                          int64_t ld, int cbits, T* __restrict__ out) {
+  using K = typename KeyOf<T>::type;
+  extern __shared__ __align__(8) unsigned char lds[];
+  K* tile = (K*)lds;  // [column][row], odd pitch
+  const int n = (int)nrow, pitch = n | 1, C = 1 << cbits;
+  const int64_t c0 = (int64_t)blockIdx.x << cbits;
+  const int cq = threadIdx.x & (C - 1), rstep = 256 >> cbits;
+  if (c0 + cq < ncol) {
+    const T* p = dat + c0 + cq;
+#pragma unroll 8
+    for (int i = threadIdx.x >> cbits; i < n; i += rstep) tile[cq * pitch + i] = order_key(p[(int64_t)i * ld]);
   }
-  // bitonic sort of index i = e * 64 + lane, ascending
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const int ncl = (int)min((int64_t)C, ncol - c0);
+  const int k = (n - 1) / 2;  // the lower middle value
+  for (int c = threadIdx.x >> 6; c < ncl; c += 4) {
+    K x[V];
+    K mn = ~(K)0, mx = 0;
 #pragma unroll
-  for (int k = 2; k <= N; k <<= 1) {
+    for (int e = 0; e < V; e++) {
+      const int i = e * kWave + lane;
+      const bool in = i < n;
+      x[e] = in ? tile[c * pitch + i] : ~(K)0;  // the padding counts only above every pivot
+      mn = min(mn, x[e]);
+      mx = max(mx, in ? x[e] : (K)0);
+    }
+    K lo = wave_min(mn), hi = ~wave_min((K)~mx);  // x_k is in [lo, hi]
+    int clo = 0, chi = n;                         // keys below lo, keys up to hi
+    while (lo < hi && chi - clo > 1) {
+      const K mid = lo + (hi - lo) / 2;
+      int cnt = 0;
 #pragma unroll
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      if (j >= kWave) {  // partner in the same lane: register e ^ (j / 64)
-        const int jj = j / kWave;
-#pragma unroll
-        for (int e = 0; e < V; e++) {
-          if (e & jj) continue;
-          const int i = e * kWave + lane;
-          const bool up = (i & k) == 0;
-          const T a = x[e], b = x[e ^ jj];
-          const T lo = a < b ? a : b, hi = a < b ? b : a;
-          x[e] = up ? lo : hi;
-          x[e ^ jj] = up ? hi : lo;
-        }
-      } else {  // partner in lane ^ j, same register
-#pragma unroll
-        for (int e = 0; e < V; e++) {
-          const int i = e * kWave + lane;
-          const T y = __shfl_xor(x[e], j, 64);
-          const bool up = (i & k) == 0, lower = (i & j) == 0;
-          const T lo = x[e] < y ? x[e] : y, hi = x[e] < y ? y : x[e];
-          x[e] = (up == lower) ? lo : hi;
-        }
+      for (int e = 0; e < V; e++) cnt += __popcll(__ballot(x[e] <= mid));
+      if (cnt > k) {
+        hi = mid;
+        chi = cnt;
+      } else {
+        lo = mid + 1;
+        clo = cnt;
       }
     }
-  }
-  auto at = [&](int64_t i) -> T {  // sorted element i (uniform index)
-    const int e = (int)(i / kWave), l = (int)(i % kWave);
-    T v = x[0];
+    K a = hi;
+    if (lo < hi) {  // the one key in the bracket
+      a = ~(K)0;
 #pragma unroll
-    for (int q = 1; q < V; q++)
-      if (q == e) v = x[q];
-    return __shfl(v, l, 64);
-  };
-  T med;
-  if (nrow & 1) {
-    med = at((nrow - 1) / 2);
-  } else {
-    const T a = at(nrow / 2 - 1), b = at(nrow / 2);
-    med = (a + b) / T(2);
+      for (int e = 0; e < V; e++) a = min(a, x[e] >= lo ? x[e] : ~(K)0);
+      a = wave_min(a);
+    }
+    T med = key_value(a);
+    if (!(n & 1)) {
+      K b = a;
+      if (chi < k + 2) {  // the next value up is another one
+        b = ~(K)0;
+#pragma unroll
+        for (int e = 0; e < V; e++) b = min(b, x[e] > a ? x[e] : ~(K)0);
+        b = wave_min(b);
+      }
+      med = (med + key_value(b)) / T(2);
+    }
+    if (lane == 0) out[c0 + c] = med;
   }
-  if (lane == 0) out[c] = med;
 }
 
 template <typename T>
@@ -116,37 +165,58 @@ __global__ void __launch_bounds__(256) design_kernel(const T* __restrict__ cm, i
   }
 }
 
-constexpr int kDotChunk = 8192;  // samples per partial
+constexpr int kDotChunk = 4096;  // samples per partial
 constexpr int kMaxCol = 8;
+constexpr int kDotRows = 8;      // rows per workgroup
 
-// part[(j * nchunk + chunk) * ncol + k] = sum over the chunk of X[t][k] y_j[t]
-template <typename T>
-__global__ void __launch_bounds__(256) design_dots_kernel(const double* __restrict__ X, int64_t n, int ncol,
-                                                          const T* __restrict__ y, int64_t ld, int64_t nchunk,
-                                                          double* __restrict__ part) {
-  __shared__ double red[kMaxCol][256];
-  const int64_t j = blockIdx.y, chunk = blockIdx.x;
+// part[(j * nchunk + chunk) * ncol + k] = sum over the chunk of X[t][k] y_j[t].
+// Bandwidth-bound on y: a thread holds one sample's NC design values and
+// applies them to kDotRows rows, so the FP64 design, twice as wide as a FP32
+// row per column, is read once per 8 rows instead of once per row.  The 8 x NC
+// sums of a thread are halved and exchanged lane by lane, after which lane l
+// holds sum l of the wave (63 exchanges instead of 6 per sum).  215 rows x
+// 100003, NC = 6, FP32: 47 us from 247 us (a row per workgroup).
+template <typename T, int NC>
+__global__ void __launch_bounds__(256) design_dots_kernel(const double* __restrict__ X, int64_t n,
+                                                          const T* __restrict__ y, int64_t nrow, int64_t ld,
+                                                          int64_t nchunk, double* __restrict__ part) {
+  __shared__ double red[4][64];
+  const int64_t j0 = (int64_t)blockIdx.y * kDotRows, chunk = blockIdx.x;
   const int64_t t0 = chunk * kDotChunk, t1 = min(n, t0 + kDotChunk);
-  double acc[kMaxCol];
+  const int nr = (int)min((int64_t)kDotRows, nrow - j0);
+  double acc[64];
 #pragma unroll
-  for (int k = 0; k < kMaxCol; k++) acc[k] = 0.0;
-  const T* row = y + j * ld;
-  for (int64_t t = t0 + threadIdx.x; t < t1; t += blockDim.x) {
-    const double v = (double)row[t];
+  for (int e = 0; e < 64; e++) acc[e] = 0.0;
+  const T* rows = y + j0 * ld;
+#pragma unroll 2
+  for (int64_t t = t0 + threadIdx.x; t < t1; t += 256) {
+    double xv[NC];
+    T v[kDotRows];
 #pragma unroll
-    for (int k = 0; k < kMaxCol; k++)
-      if (k < ncol) acc[k] += X[t * ncol + k] * v;
+    for (int r = 0; r < kDotRows; r++) v[r] = r < nr ? rows[r * ld + t] : T(0);
+#pragma unroll
+    for (int k = 0; k < NC; k++) xv[k] = X[t * NC + k];
+#pragma unroll
+    for (int r = 0; r < kDotRows; r++)
+#pragma unroll
+      for (int k = 0; k < NC; k++) acc[r * 8 + k] += xv[k] * (double)v[r];
   }
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
-  for (int k = 0; k < kMaxCol; k++) red[k][threadIdx.x] = acc[k];
+  for (int h = 32; h; h >>= 1) {
+    const bool up = lane & h;
+#pragma unroll
+    for (int e = 0; e < h; e++) {
+      const double keep = up ? acc[e + h] : acc[e], give = up ? acc[e] : acc[e + h];
+      acc[e] = keep + __shfl_xor(give, h, 64);
+    }
+  }
+  red[wave][lane] = acc[0];
   __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s)
-#pragma unroll
-      for (int k = 0; k < kMaxCol; k++) red[k][threadIdx.x] += red[k][threadIdx.x + s];
-    __syncthreads();
-  }
-  if ((int)threadIdx.x < ncol) part[(j * nchunk + chunk) * ncol + threadIdx.x] = red[threadIdx.x][0];
+  const int r = threadIdx.x >> 3, k = threadIdx.x & 7;
+  if (r < nr && k < NC)
+    part[((j0 + r) * nchunk + chunk) * NC + k] = ((red[0][threadIdx.x] + red[1][threadIdx.x]) + red[2][threadIdx.x]) +
+                                                 red[3][threadIdx.x];
 }
 
 // D[k][j] = sum over chunks (in order) of the partials
@@ -156,22 +226,41 @@ __global__ void design_dots_reduce(const double* __restrict__ part, int64_t nrow
        e += (int64_t)gridDim.x * blockDim.x) {
     const int64_t j = e / ncol, k = e % ncol;
     double s = 0.0;
+#pragma unroll 8
     for (int64_t c = 0; c < nchunk; c++) s += part[(j * nchunk + c) * ncol + k];
     D[k * nrow + j] = s;
   }
 }
 
-template <typename T>
+// Bandwidth-bound on base and out: a thread holds one sample's NK design
+// values and applies them to kDotRows rows, whose coefficients are scalar.
+// 215 x 100003, NK = 3, FP32: 50 us (3.4 TB/s) from 120 us (one element per thread and
+// step, the design read again for every row).  NK < 0: more than kMaxCol
+// columns, read as they are used.
+template <typename T, int NK>
 __global__ void __launch_bounds__(256) design_apply_kernel(const T* __restrict__ base, int64_t nrow, int64_t n,
                                                            int64_t ld, const double* __restrict__ X, int ncol, int c0,
-                                                           int nk, const double* __restrict__ coef, T* __restrict__ out,
-                                                           int64_t ld_out) {
-  const int64_t total = nrow * n;
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t j = e / n, t = e - j * n;
+                                                           int nk, const double* __restrict__ coef,
+                                                           T* __restrict__ out, int64_t ld_out, int64_t ntile) {
+  const int64_t jg = blockIdx.x / ntile, t = (blockIdx.x - jg * ntile) * 256 + threadIdx.x;
+  if (t >= n) return;
+  const int64_t j0 = jg * kDotRows;
+  const int nr = (int)min((int64_t)kDotRows, nrow - j0);
+  double xv[NK > 0 ? NK : 1];
+#pragma unroll
+  for (int k = 0; k < NK; k++) xv[k] = X[t * ncol + c0 + k];
+  T v[kDotRows];
+#pragma unroll
+  for (int r = 0; r < kDotRows; r++) v[r] = base && r < nr ? base[(j0 + r) * ld + t] : T(0);
+#pragma unroll
+  for (int r = 0; r < kDotRows; r++) {
+    if (r >= nr) break;
     double p = 0.0;
-    for (int k = 0; k < nk; k++) p += X[t * ncol + c0 + k] * coef[k * nrow + j];
-    out[j * ld_out + t] = base ? (T)((double)base[j * ld + t] - p) : (T)p;
+#pragma unroll
+    for (int k = 0; k < NK; k++) p += xv[k] * coef[k * nrow + j0 + r];
+    if constexpr (NK < 0)
+      for (int k = 0; k < nk; k++) p += X[t * ncol + c0 + k] * coef[k * nrow + j0 + r];
+    out[(j0 + r) * ld_out + t] = base ? (T)((double)v[r] - p) : (T)p;
   }
 }
 
@@ -182,13 +271,20 @@ int median_cols_impl(const T* dat, int64_t nrow, int64_t ncol, int64_t ld, T* ou
              (long long)ld);
   if (ncol == 0) return MK_OK;
   MK_REQUIRE(dat && out, MK_ERR_ARG, "null pointer");
-  const unsigned grid = (unsigned)mk::cdiv(ncol, 4);
+  // columns per workgroup: 32 where they fit 20 KB (eight workgroups a CU),
+  // fewer for tall blocks
+  int cbits = 5;
+  while (cbits > 2 && (((size_t)(nrow | 1) * sizeof(T)) << cbits) > 20 * 1024) cbits--;
+  const size_t lds = ((size_t)(nrow | 1) * sizeof(T)) << cbits;
+  const int64_t groups = mk::cdiv(ncol, (int64_t)1 << cbits);
+  MK_REQUIRE(groups < INT32_MAX, MK_ERR_ARG, "median: too many columns");
+  const unsigned grid = (unsigned)groups;
   hipStream_t st = mk::as_stream(stream);
-  if (nrow <= 64) median_cols_kernel<T, 1><<<grid, 256, 0, st>>>(dat, nrow, ncol, ld, out);
-  else if (nrow <= 128) median_cols_kernel<T, 2><<<grid, 256, 0, st>>>(dat, nrow, ncol, ld, out);
-  else if (nrow <= 256) median_cols_kernel<T, 4><<<grid, 256, 0, st>>>(dat, nrow, ncol, ld, out);
-  else if (nrow <= 512) median_cols_kernel<T, 8><<<grid, 256, 0, st>>>(dat, nrow, ncol, ld, out);
-  else median_cols_kernel<T, 16><<<grid, 256, 0, st>>>(dat, nrow, ncol, ld, out);
+  if (nrow <= 64) median_cols_kernel<T, 1><<<grid, 256, lds, st>>>(dat, nrow, ncol, ld, cbits, out);
+  else if (nrow <= 128) median_cols_kernel<T, 2><<<grid, 256, lds, st>>>(dat, nrow, ncol, ld, cbits, out);
+  else if (nrow <= 256) median_cols_kernel<T, 4><<<grid, 256, lds, st>>>(dat, nrow, ncol, ld, cbits, out);
+  else if (nrow <= 512) median_cols_kernel<T, 8><<<grid, 256, lds, st>>>(dat, nrow, ncol, ld, cbits, out);
+  else median_cols_kernel<T, 16><<<grid, 256, lds, st>>>(dat, nrow, ncol, ld, cbits, out);
   return mk::check_launch("median_cols_kernel");
 }
 
@@ -210,8 +306,14 @@ int dots_impl(const double* X, int64_t n, int ncol, const T* y, int64_t nrow, in
   const int64_t nchunk = mk::cdiv(n, kDotChunk);
   MK_REQUIRE(work_bytes >= nrow * nchunk * ncol * 8, MK_ERR_ARG, "workspace too small");
   hipStream_t st = mk::as_stream(stream);
-  design_dots_kernel<T><<<dim3((unsigned)nchunk, (unsigned)nrow), 256, 0, st>>>(X, n, ncol, y, ld, nchunk,
-                                                                               (double*)work);
+  const dim3 grid((unsigned)nchunk, (unsigned)mk::cdiv(nrow, kDotRows));
+  double* part = (double*)work;
+  switch (ncol) {
+#define MK_DOTS(NC) \
+  case NC: design_dots_kernel<T, NC><<<grid, 256, 0, st>>>(X, n, y, nrow, ld, nchunk, part); break
+    MK_DOTS(1); MK_DOTS(2); MK_DOTS(3); MK_DOTS(4); MK_DOTS(5); MK_DOTS(6); MK_DOTS(7); MK_DOTS(8);
+#undef MK_DOTS
+  }
   int r = mk::check_launch("design_dots_kernel");
   if (r) return r;
   design_dots_reduce<<<mk::grid_for(nrow * ncol, 256), 256, 0, st>>>((const double*)work, nrow, ncol, nchunk, D);
@@ -225,8 +327,19 @@ int apply_impl(const T* base, int64_t nrow, int64_t n, int64_t ld, const double*
              MK_ERR_ARG, "bad design apply sizes");
   if (nrow == 0) return MK_OK;
   MK_REQUIRE(X && coef && out, MK_ERR_ARG, "null pointer");
-  design_apply_kernel<T><<<mk::grid_for(nrow * n, 256, 256 * 64), 256, 0, mk::as_stream(stream)>>>(
-      base, nrow, n, ld, X, ncol, c0, nk, coef, out, ld_out);
+  const int64_t ntile = mk::cdiv(n, 256), groups = ntile * mk::cdiv(nrow, kDotRows);
+  MK_REQUIRE(groups < INT32_MAX, MK_ERR_ARG, "bad design apply sizes");
+  hipStream_t st = mk::as_stream(stream);
+  switch (nk) {
+#define MK_APPLY(LABEL, NK)                                                                                      \
+  LABEL:                                                                                                         \
+    design_apply_kernel<T, NK><<<(unsigned)groups, 256, 0, st>>>(base, nrow, n, ld, X, ncol, c0, nk, coef, out,  \
+                                                                 ld_out, ntile);                                 \
+    break
+    MK_APPLY(case 0, 0); MK_APPLY(case 1, 1); MK_APPLY(case 2, 2); MK_APPLY(case 3, 3); MK_APPLY(case 4, 4);
+    MK_APPLY(case 5, 5); MK_APPLY(case 6, 6); MK_APPLY(case 7, 7); MK_APPLY(case 8, 8); MK_APPLY(default, -1);
+#undef MK_APPLY
+  }
   return mk::check_launch("design_apply_kernel");
 }
 

@@ -129,24 +129,25 @@ def fit_cm_plus_poly(dat, ord=2, cm_ord=1, niter=1, medsub=False, full_out=False
         raise ValueError("ord + 1 + cm_ord must be at most 8")
     f64 = dict(dtype=torch.float64, device=d.device)
     sp = dev.stream_ptr()
-    dd = d.clone()
+    dd = torch.empty_like(d) if niter > 0 else d.clone()
     cm = torch.zeros(n, dtype=d.dtype, device=d.device)
     pred2 = torch.zeros(n, dtype=d.dtype, device=d.device)  # the reference's initial value (niter = 0)
     X = torch.empty((n, ncol), **f64)
     Xt = torch.empty((ncol, n), **f64)
-    lhs = torch.empty((ncol, ncol), **f64)
-    rhs = torch.empty((ncol, ndet), **f64)
+    normal = torch.empty(ncol * (ncol + ndet), **f64)  # left and right sides, fetched in one copy
+    lhs, rhs = normal[:ncol * ncol], normal[ncol * ncol:]
     wb = max(int(mkgpu.lib.mk_design_dots_workspace_bytes(n, ncol, ndet)),
              int(mkgpu.lib.mk_design_dots_workspace_bytes(n, ncol, ncol)))
     work = torch.empty(wb // 8 + 32, **f64)
-    for _ in range(niter):
-        mkgpu.check("mk_median_cols_" + sfx, dd.data_ptr(), ndet, n, n, cm.data_ptr(), sp)
+    for it in range(niter):
+        mkgpu.check("mk_median_cols_" + sfx, (dd if it else d).data_ptr(), ndet, n, n, cm.data_ptr(), sp)
         mkgpu.check("mk_cm_poly_design_" + sfx, cm.data_ptr(), n, ord, cm_ord, X.data_ptr(), Xt.data_ptr(), sp)
         mkgpu.check("mk_design_dots_f64", X.data_ptr(), n, ncol, Xt.data_ptr(), ncol, n, lhs.data_ptr(),
                     work.data_ptr(), work.numel() * 8, sp)
         mkgpu.check("mk_design_dots_" + sfx, X.data_ptr(), n, ncol, d.data_ptr(), ndet, n, rhs.data_ptr(),
                     work.data_ptr(), work.numel() * 8, sp)
-        fitp = np.dot(np.linalg.inv(lhs.cpu().numpy()), rhs.cpu().numpy())
+        sides = normal.cpu().numpy()
+        fitp = np.dot(np.linalg.inv(sides[:ncol * ncol].reshape(ncol, ncol)), sides[ncol * ncol:].reshape(ncol, ndet))
         coef = torch.from_numpy(np.ascontiguousarray(fitp)).to(d.device)
         mkgpu.check("mk_design_apply_" + sfx, d.data_ptr(), ndet, n, n, X.data_ptr(), ncol, 0, ord + 1,
                     coef.data_ptr(), dd.data_ptr(), n, sp)

@@ -95,3 +95,73 @@ def test_downsample_tod_matches_oracle(env):
     d32 = {"dat_calib": device.to_device(dat.astype(np.float32)), "dt": 1.0}
     downsample_tod(d32, 4)
     assert rel_err(d32["dat_calib"].cpu().numpy(), opre.downsample_array(dat.astype(np.float32), 4)) < 2e-6
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("nrow", [1, 2, 5, 64, 130, 700, 1024])
+def test_median_cols_extreme_values(env, dtype, nrow):
+    """Infinities, equal values, zeros of both signs, subnormals, and a range
+    that spans every exponent: the order statistics are exact."""
+    torch, device, mkgpu = env
+    rng = np.random.default_rng(nrow)
+    tiny = np.finfo(dtype).tiny
+    a = rng.standard_normal((nrow, 33)).astype(dtype)
+    a[:, 0] = 3.25
+    a[:, 1] = np.inf
+    a[:, 2] = -np.inf
+    a[: nrow // 3, 3] = np.inf
+    a[: nrow // 3, 4] = -np.inf
+    a[:, 5] = np.where(np.arange(nrow) % 2, 0.0, -0.0)
+    a[:, 6] = rng.integers(-3, 4, nrow) * (tiny / 4)
+    a[:, 7] = rng.integers(0, 2, nrow)
+    a[:, 8] = np.exp(rng.uniform(-80, 80, nrow)) * rng.choice([-1, 1], nrow)
+    a[:, 9] = -np.abs(a[:, 9])
+    at = device.to_device(a)
+    out = torch.empty(33, dtype=at.dtype, device=at.device)
+    print("median", dtype.__name__, nrow, flush=True)
+    mkgpu.check("mk_median_cols_" + ("f64" if dtype == np.float64 else "f32"), at.data_ptr(), nrow, 33, 33,
+                out.data_ptr(), device.stream_ptr())
+    srt = np.sort(a, axis=0)
+    ref = srt[nrow // 2] if nrow % 2 else (srt[nrow // 2 - 1] + srt[nrow // 2]) / dtype(2)
+    got = out.cpu().numpy()
+    assert np.array_equal(got[[0, 1, 2, 3, 4, 5, 7, 8, 9]], ref[[0, 1, 2, 3, 4, 5, 7, 8, 9]])
+    assert abs(got[6] - ref[6]) <= tiny / 8  # the halved sum of an odd subnormal sum rounds to either side
+    assert np.array_equal(got[10:], ref[10:])
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("nrow,n,ncol", [(1, 1, 1), (7, 255, 2), (8, 256, 3), (9, 257, 5), (17, 4096, 6), (5, 4097, 7),
+                                         (16, 9001, 8), (3, 300, 11)])
+def test_design_dots_and_apply_edges(env, dtype, nrow, n, ncol):
+    """Row groups of 8 and sample chunks of 256 and 4096 with remainders.
+    FP64 sums: n eps of the sum of magnitudes (1e-12); the subtraction rounds
+    once more in the data type."""
+    torch, device, mkgpu = env
+    sfx = "f64" if dtype == np.float64 else "f32"
+    rng = np.random.default_rng(nrow + n + ncol)
+    X, ld = rng.standard_normal((n, ncol)), n + 5
+    y = rng.standard_normal((nrow, ld)).astype(dtype)
+    Xt, yt = device.to_device(X), device.to_device(y)
+    f64 = dict(dtype=torch.float64, device=yt.device)
+    sp = device.stream_ptr()
+    print("design", sfx, nrow, n, ncol, flush=True)
+    if ncol <= 8:
+        nb = int(mkgpu.lib.mk_design_dots_workspace_bytes(n, ncol, nrow))
+        work, D = torch.empty(nb // 8, **f64), torch.empty((ncol, nrow), **f64)
+        mkgpu.check("mk_design_dots_" + sfx, Xt.data_ptr(), n, ncol, yt.data_ptr(), nrow, ld, D.data_ptr(),
+                    work.data_ptr(), nb // 8 * 8, sp)
+        ref = X.T @ y[:, :n].astype(np.float64).T
+        assert np.all(np.abs(D.cpu().numpy() - ref) <= 1e-12 * (np.abs(X.T) @ np.abs(y[:, :n].astype(np.float64).T)))
+    c0 = min(1, ncol - 1)
+    coef = rng.standard_normal((ncol - c0, nrow))
+    ct = device.to_device(coef)
+    p = (X[:, c0:] @ coef).T
+    eps = np.finfo(dtype).eps
+    for base in (True, False):
+        out = torch.full((nrow, n + 2), 9.0, dtype=yt.dtype, device=yt.device)
+        mkgpu.check("mk_design_apply_" + sfx, yt.data_ptr() if base else 0, nrow, n, ld, Xt.data_ptr(), ncol, c0,
+                    ncol - c0, ct.data_ptr(), out.data_ptr(), n + 2, sp)
+        ref = y[:, :n].astype(np.float64) - p if base else p
+        got = out.cpu().numpy()
+        assert np.all(got[:, n:] == 9.0)
+        assert np.all(np.abs(got[:, :n] - ref) <= eps * (np.abs(ref) + 20 * np.finfo(np.float64).eps / eps * 100))
