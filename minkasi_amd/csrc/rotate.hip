@@ -467,100 +467,189 @@ __global__ void split_matrix_kernel(const double* __restrict__ a, int64_t M, int
 // ---------------------------------------------------------------------------
 // FP64 setup GEMMs
 
-constexpr int TB = 64, TK = 16;
+// v_mfma_f64_16x16x4f64: lane l holds A[l % 16][l / 16], B[l / 16][l % 16] and
+// D[4 r + l / 16][l % 16] in register r.  The products of a step may be summed
+// in any order, so lane l carries the four consecutive k of quarter l / 16 of a
+// 16-deep step (one wide load along a row) and step c multiplies the c-th of
+// every quarter.
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+constexpr int TK = 16;
 
-// C[M x N] = A[M x K] . B[K x N]; A FP64 row-major (lda), B of type TB_ (ldb),
-// C FP64 (ldc).  64x64 tile per workgroup, 4x4 per thread.
+template <typename T>
+struct alignas(sizeof(T)) Row4 { T v[4]; };  // four elements at element alignment
+
+__device__ __forceinline__ f64x4 mfma_f64(double a, double b, f64x4 c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+// p[0..3] as FP64 where k + e < kend, else 0.
+template <typename T>
+__device__ __forceinline__ f64x4 load4(const T* __restrict__ p, int64_t left) {
+  f64x4 r;
+  if (left >= 4) {
+    const Row4<T> q = *reinterpret_cast<const Row4<T>*>(p);
+#pragma unroll
+    for (int e = 0; e < 4; e++) r[e] = (double)q.v[e];
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; e++) r[e] = e < left ? (double)p[e] : 0.0;
+  }
+  return r;
+}
+
+// C[M x N] = A[M x K] . B[K x N]; A FP64 row-major (lda), B of type TBT (ldb),
+// C FP64 (ldc).  Bound by the matrix cores, whose FP64 rate is the vector
+// unit's, but which take their operands once per 16 products: a wave owns 32 x
+// 64 of C and reads both operands from memory into the fragments (B in rows of
+// 64 columns, lane l the columns 4 (l % 16) + j of tile j; A is small and stays
+// in the caches), loading a step ahead.  rw of the workgroup's 4 waves go down
+// the rows, so that they share B's lines.  215 x 215 x 90001, B FP32: 308 us
+// from 375 (64 x 64 tiles through LDS on the vector unit); 64 x 64 x 65536,
+// FP64: 24 us from 34.
 template <typename TBT>
 __global__ void __launch_bounds__(256) gemm_nn_f64(int M, int N, int K, const double* __restrict__ A, int64_t lda,
                                                    const TBT* __restrict__ B, int64_t ldb, double* __restrict__ C,
-                                                   int64_t ldc) {
-  __shared__ double As[TK][TB + 1];
-  __shared__ double Bs[TK][TB + 1];
-  const int bm = blockIdx.y * TB, bn = blockIdx.x * TB;
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  double acc[4][4] = {};
+                                                   int64_t ldc, int rw) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int m0 = ((int)blockIdx.y * rw + wave % rw) * 32, n0 = ((int)blockIdx.x * (4 / rw) + wave / rw) * 64;
+  if (m0 >= M || n0 >= N) return;
+  const int lr = lane & 15, lk = 4 * (lane >> 4);
+  const double* a0 = A + (int64_t)min(m0 + lr, M - 1) * lda + lk;       // rows past M repeat the last one
+  const double* a1 = A + (int64_t)min(m0 + 16 + lr, M - 1) * lda + lk;  // and are not stored
+  const int nc = n0 + 4 * lr;
+  const TBT* b0 = B + nc;
+  const int nleft = N - nc;  // columns from this lane's first one
+  f64x4 acc[2][4];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 4; j++) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
+  auto load = [&](int k0, f64x4& x0, f64x4& x1, f64x4 (&y)[4]) {
+    x0 = load4(a0 + k0, K - k0 - lk);
+    x1 = load4(a1 + k0, K - k0 - lk);
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      const int k = k0 + lk + c;
+      y[c] = load4(b0 + (int64_t)min(k, K - 1) * ldb, k < K ? nleft : 0);
+    }
+  };
+  f64x4 x0, x1, y[4], p0, p1, q[4];
+  load(0, x0, x1, y);
   for (int k0 = 0; k0 < K; k0 += TK) {
-    for (int idx = threadIdx.x; idx < TK * TB; idx += 256) {
-      int kk = idx / TB, mm = idx % TB;
-      int gm = bm + mm, gk = k0 + kk;
-      As[kk][mm] = (gm < M && gk < K) ? A[(int64_t)gm * lda + gk] : 0.0;
-      int gn = bn + mm;
-      Bs[kk][mm] = (gk < K && gn < N) ? (double)B[(int64_t)gk * ldb + gn] : 0.0;
+    const bool more = k0 + TK < K;
+    if (more) load(k0 + TK, p0, p1, q);
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        acc[0][j] = mfma_f64(x0[c], y[c][j], acc[0][j]);
+        acc[1][j] = mfma_f64(x1[c], y[c][j], acc[1][j]);
+      }
+    if (more) {
+      x0 = p0;
+      x1 = p1;
+#pragma unroll
+      for (int c = 0; c < 4; c++) y[c] = q[c];
     }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < TK; kk++) {
-      double a[4], b[4];
-#pragma unroll
-      for (int i = 0; i < 4; i++) a[i] = As[kk][ty + 16 * i];
-#pragma unroll
-      for (int j = 0; j < 4; j++) b[j] = Bs[kk][tx + 16 * j];
-#pragma unroll
-      for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j] = fma(a[i], b[j], acc[i][j]);
-    }
-    __syncthreads();
   }
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+  for (int i = 0; i < 2; i++)
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      int gm = bm + ty + 16 * i, gn = bn + tx + 16 * j;
-      if (gm < M && gn < N) C[(int64_t)gm * ldc + gn] = acc[i][j];
+    for (int r = 0; r < 4; r++) {
+      const int gm = m0 + 16 * i + 4 * r + (lane >> 4);
+      if (gm >= M) continue;
+      double* out = C + (int64_t)gm * ldc + nc;
+      if (nleft >= 4) {
+        *reinterpret_cast<Row4<double>*>(out) = {acc[i][0][r], acc[i][1][r], acc[i][2][r], acc[i][3][r]};
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          if (j < nleft) out[j] = acc[i][j][r];
+      }
     }
 }
 
 // Partial cross products over chunks of the long axis:
 // P[chunk][M x N] = A[:, chunk] . B[:, chunk]^T (A: M rows, B: N rows, both
-// row-major with n columns; the Gram matrix is A = B).
-template <typename TA, typename TB2>
+// row-major with n columns; the Gram matrix is A = B).  Bound by the matrix
+// cores like gemm_nn_f64: a workgroup owns 64 x 64, a wave 32 x 32 of it, and
+// both operands are read along their rows into the fragments.  SYM: A = B, and
+// only the tiles on and above the diagonal are computed; their mirror images
+// are the same sums.  Gram of 215 x 90001 FP32: 372 us from 1979 (64 x 64 tiles
+// through LDS on the vector unit, all tiles, 176 workgroups).
+constexpr int TB = 64;
+
+template <typename TA, typename TB2, bool SYM>
 __global__ void __launch_bounds__(256) cross_partial_f64(int M, int N, int64_t n, const TA* __restrict__ A,
                                                          int64_t lda, const TB2* __restrict__ B, int64_t ldb,
                                                          int64_t chunk, double* __restrict__ P) {
-  __shared__ double As[TK][TB + 1];
-  __shared__ double Bs[TK][TB + 1];
-  const int bm = blockIdx.y * TB, bn = blockIdx.x * TB;
+  if (SYM && blockIdx.x < blockIdx.y) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int bm = (int)blockIdx.y * TB + 32 * (wave & 1), bn = (int)blockIdx.x * TB + 32 * (wave >> 1);
+  if (bm >= M || bn >= N) return;
   const int64_t c0 = (int64_t)blockIdx.z * chunk, c1 = min(n, c0 + chunk);
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  double acc[4][4] = {};
+  const int lr = lane & 15, lk = 4 * (lane >> 4);
+  const TA* a[2] = {A + (int64_t)min(bm + lr, M - 1) * lda + lk, A + (int64_t)min(bm + 16 + lr, M - 1) * lda + lk};
+  const TB2* b[2] = {B + (int64_t)min(bn + lr, N - 1) * ldb + lk, B + (int64_t)min(bn + 16 + lr, N - 1) * ldb + lk};
+  f64x4 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
+  auto load = [&](int64_t k0, f64x4 (&x)[2], f64x4 (&y)[2]) {
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      x[i] = load4(a[i] + k0, c1 - k0 - lk);
+      y[i] = load4(b[i] + k0, c1 - k0 - lk);
+    }
+  };
+  f64x4 x[2], y[2], p[2], q[2];
+  load(c0, x, y);
   for (int64_t k0 = c0; k0 < c1; k0 += TK) {
-    for (int idx = threadIdx.x; idx < TK * TB; idx += 256) {
-      int mm = idx / TK, kk = idx % TK;  // consecutive threads walk along n
-      int64_t gk = k0 + kk;
-      int gm = bm + mm, gn = bn + mm;
-      As[kk][mm] = (gm < M && gk < c1) ? (double)A[(int64_t)gm * lda + gk] : 0.0;
-      Bs[kk][mm] = (gn < N && gk < c1) ? (double)B[(int64_t)gn * ldb + gk] : 0.0;
+    const bool more = k0 + TK < c1;
+    if (more) load(k0 + TK, p, q);
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[i][j] = mfma_f64(x[i][c], y[j][c], acc[i][j]);
+    if (more) {
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        x[i] = p[i];
+        y[i] = q[i];
+      }
     }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < TK; kk++) {
-      double a[4], b[4];
-#pragma unroll
-      for (int i = 0; i < 4; i++) a[i] = As[kk][ty + 16 * i];
-#pragma unroll
-      for (int j = 0; j < 4; j++) b[j] = Bs[kk][tx + 16 * j];
-#pragma unroll
-      for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j] = fma(a[i], b[j], acc[i][j]);
-    }
-    __syncthreads();
   }
   double* out = P + (int64_t)blockIdx.z * M * N;
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+  for (int i = 0; i < 2; i++)
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      int gm = bm + ty + 16 * i, gn = bn + tx + 16 * j;
-      if (gm < M && gn < N) out[(int64_t)gm * N + gn] = acc[i][j];
-    }
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int gm = bm + 16 * i + 4 * r + (lane >> 4), gn = bn + 16 * j + lr;
+        if (gm >= M || gn >= N) continue;
+        out[(int64_t)gm * N + gn] = acc[i][j][r];
+        if (SYM && blockIdx.x > blockIdx.y) out[(int64_t)gn * N + gm] = acc[i][j][r];
+      }
+}
+
+// Samples per partial: at most 8192 (a partial costs M x N FP64 numbers of
+// workspace), down to 1024 while the tiles alone leave the chip short of two
+// workgroups per CU.  215 x 90001: 1024 gives 880 workgroups, 8192 gave 110.
+int64_t cross_chunk(int64_t M, int64_t N, int64_t n, bool sym) {
+  const int64_t tm = mk::cdiv(M, TB), tiles = sym ? tm * (tm + 1) / 2 : tm * mk::cdiv(N, TB);
+  int64_t chunk = 8192;
+  while (chunk > 1024 && tiles * mk::cdiv(n, chunk) < 512) chunk /= 2;
+  return chunk;
 }
 
 __global__ void sum_partials_f64(const double* __restrict__ P, int64_t nchunk, int64_t mm, double* __restrict__ G) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < mm; i += (int64_t)gridDim.x * blockDim.x) {
     double s = 0.0;
+#pragma unroll 8
     for (int64_t c = 0; c < nchunk; c++) s += P[c * mm + i];
     G[i] = s;
   }
@@ -697,45 +786,48 @@ extern "C" int mk_gemm_nn_f64(int64_t M, int64_t N, int64_t K, const double* A, 
   MK_REQUIRE(M > 0 && N >= 0 && K > 0 && A && B && C, MK_ERR_ARG, "bad arguments");
   if (N == 0) return MK_OK;
   MK_REQUIRE(M < 65536 * TB, MK_ERR_ARG, "M too large");
-  dim3 grid((unsigned)mk::cdiv(N, TB), (unsigned)mk::cdiv(M, TB));
+  const int rw = M <= 32 ? 1 : M <= 64 ? 2 : 4;  // waves down the rows
+  dim3 grid((unsigned)mk::cdiv(N, 64 * (4 / rw)), (unsigned)mk::cdiv(M, 32 * rw));
   hipStream_t st = mk::as_stream(stream);
   if (b_is_f32)
-    gemm_nn_f64<float><<<grid, 256, 0, st>>>((int)M, (int)N, (int)K, A, lda, (const float*)B, ldb, C, ldc);
+    gemm_nn_f64<float><<<grid, 256, 0, st>>>((int)M, (int)N, (int)K, A, lda, (const float*)B, ldb, C, ldc, rw);
   else
-    gemm_nn_f64<double><<<grid, 256, 0, st>>>((int)M, (int)N, (int)K, A, lda, (const double*)B, ldb, C, ldc);
+    gemm_nn_f64<double><<<grid, 256, 0, st>>>((int)M, (int)N, (int)K, A, lda, (const double*)B, ldb, C, ldc, rw);
   return mk::check_launch("gemm_nn_f64");
 }
 
-extern "C" int64_t mk_gram_workspace_bytes(int64_t M, int64_t n) {
-  int64_t chunk = 8192;
-  int64_t nchunk = std::max<int64_t>(1, mk::cdiv(n, chunk));
-  return nchunk * M * M * 8 + 256;
+namespace {
+int64_t cross_work_bytes(int64_t M, int64_t N, int64_t n, bool sym) {
+  return std::max<int64_t>(1, mk::cdiv(n, cross_chunk(M, N, n, sym))) * M * N * 8 + 256;
 }
+
+template <typename T, bool SYM>
+int cross_impl(int64_t M, int64_t N, int64_t n, const T* A, int64_t lda, const T* B, int64_t ldb, double* C,
+               void* work, void* stream) {
+  const int64_t chunk = cross_chunk(M, N, n, SYM), nchunk = std::max<int64_t>(1, mk::cdiv(n, chunk));
+  MK_REQUIRE(nchunk < 65536, MK_ERR_ARG, "n too large");
+  dim3 grid((unsigned)mk::cdiv(N, TB), (unsigned)mk::cdiv(M, TB), (unsigned)nchunk);
+  hipStream_t st = mk::as_stream(stream);
+  cross_partial_f64<T, T, SYM><<<grid, 256, 0, st>>>((int)M, (int)N, n, A, lda, B, ldb, chunk, (double*)work);
+  int r = mk::check_launch("cross_partial_f64");
+  if (r) return r;
+  sum_partials_f64<<<mk::grid_for(M * N, 256), 256, 0, st>>>((const double*)work, nchunk, M * N, C);
+  return mk::check_launch("sum_partials_f64");
+}
+}  // namespace
+
+extern "C" int64_t mk_gram_workspace_bytes(int64_t M, int64_t n) { return cross_work_bytes(M, M, n, true); }
 
 extern "C" int mk_gram_f64(int64_t M, int64_t n, const void* D, int d_is_f32, int64_t ldd, double* G, void* work,
                            int64_t work_bytes, void* stream) {
   MK_REQUIRE(M > 0 && n > 0 && D && G && work, MK_ERR_ARG, "bad arguments");
   MK_REQUIRE(work_bytes >= mk_gram_workspace_bytes(M, n), MK_ERR_ARG, "workspace too small");
-  int64_t chunk = 8192;
-  int64_t nchunk = std::max<int64_t>(1, mk::cdiv(n, chunk));
-  MK_REQUIRE(nchunk < 65536, MK_ERR_ARG, "n too large");
-  dim3 grid((unsigned)mk::cdiv(M, TB), (unsigned)mk::cdiv(M, TB), (unsigned)nchunk);
-  hipStream_t st = mk::as_stream(stream);
-  if (d_is_f32)
-    cross_partial_f64<float, float><<<grid, 256, 0, st>>>((int)M, (int)M, n, (const float*)D, ldd, (const float*)D,
-                                                          ldd, chunk, (double*)work);
-  else
-    cross_partial_f64<double, double><<<grid, 256, 0, st>>>((int)M, (int)M, n, (const double*)D, ldd,
-                                                            (const double*)D, ldd, chunk, (double*)work);
-  int r = mk::check_launch("cross_partial_f64");
-  if (r) return r;
-  sum_partials_f64<<<mk::grid_for(M * M, 256), 256, 0, st>>>((const double*)work, nchunk, M * M, G);
-  return mk::check_launch("sum_partials_f64");
+  return d_is_f32 ? cross_impl<float, true>(M, M, n, (const float*)D, ldd, (const float*)D, ldd, G, work, stream)
+                  : cross_impl<double, true>(M, M, n, (const double*)D, ldd, (const double*)D, ldd, G, work, stream);
 }
 
 extern "C" int64_t mk_cross_workspace_bytes(int64_t M, int64_t N, int64_t n) {
-  int64_t nchunk = std::max<int64_t>(1, mk::cdiv(n, 8192));
-  return nchunk * M * N * 8 + 256;
+  return cross_work_bytes(M, N, n, false);
 }
 
 extern "C" int mk_cross_f64(int64_t M, int64_t N, int64_t n, const double* A, int64_t lda, const double* B,
@@ -743,16 +835,7 @@ extern "C" int mk_cross_f64(int64_t M, int64_t N, int64_t n, const double* A, in
   MK_REQUIRE(M > 0 && N > 0 && n > 0 && A && B && C && work, MK_ERR_ARG, "bad arguments");
   MK_REQUIRE(M < 65536 * TB && N < 65536 * TB && lda >= n && ldb >= n, MK_ERR_ARG, "bad shapes");
   MK_REQUIRE(work_bytes >= mk_cross_workspace_bytes(M, N, n), MK_ERR_ARG, "workspace too small");
-  const int64_t chunk = 8192;
-  const int64_t nchunk = std::max<int64_t>(1, mk::cdiv(n, chunk));
-  MK_REQUIRE(nchunk < 65536, MK_ERR_ARG, "n too large");
-  dim3 grid((unsigned)mk::cdiv(N, TB), (unsigned)mk::cdiv(M, TB), (unsigned)nchunk);
-  hipStream_t st = mk::as_stream(stream);
-  cross_partial_f64<double, double><<<grid, 256, 0, st>>>((int)M, (int)N, n, A, lda, B, ldb, chunk, (double*)work);
-  int r = mk::check_launch("cross_partial_f64");
-  if (r) return r;
-  sum_partials_f64<<<mk::grid_for(M * N, 256), 256, 0, st>>>((const double*)work, nchunk, M * N, C);
-  return mk::check_launch("sum_partials_f64");
+  return cross_impl<double, false>(M, N, n, A, lda, B, ldb, C, work, stream);
 }
 
 // ---------------------------------------------------------------------------
