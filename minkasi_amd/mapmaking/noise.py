@@ -147,8 +147,9 @@ class NoiseSmoothedSVD:
         # memory (FP32), where the reference keeps its numpy array, so that it
         # does not hold 4 bytes of HBM per sample
         self.mode_wt = W.sum(dim=1).cpu().numpy()
-        self.mywt = W.to(torch.float32).cpu().numpy()
+        fetch = dev.HostFetch(W, np.float32)
         wdct = gfft._dct1_tensor(W)
+        self.mywt = fetch.result()
         del W
         self._build_apply(wdct, keep_fp64 if keep_fp64 is not None else (self.dtype == torch.float64))
 
