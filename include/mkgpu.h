@@ -287,9 +287,7 @@ int mk_pcg_set_r(float *r, const double *b, const double *ax, int64_t n,
  * Replaces many_fft_r2r_1d / many_fftf_r2r_1d (minkasi/lib/mkfftw.c:174-254,
  * bound in minkasi/lib/mkfftw.py, called by fft_r2r in
  * minkasi/tools/fft.py:290-344; scipy fallback minkasi/tools/py_fft.py:239).
- * Bluestein chirp-z on a four-step FFT of P >= 2n-1 points (FP64 rows of 1025
- * to 2^18 points: P = 2^11 q1 from a fixed list, else a power of two); any n.
- * x, y: device,
+ * Bluestein chirp-z on a power-of-two four-step FFT; any n.  x, y: device,
  * nrow*n elements; y may equal x.  work: device workspace of at least
  * mk_dct1_workspace_bytes(nrow, n, sizeof element) bytes, 256-B aligned.
  * Synchronises the stream once (descriptor upload). */
@@ -313,25 +311,23 @@ int mk_dct1_f32(const float *x, float *y, int64_t nrow, int64_t n,
 /* Noise filter y = C W C x per detector mode, C = DCT-I, W = mywt: the
  * DCT-I / weight / DCT-I core of NoiseSmoothedSVD.apply_noise
  * (minkasi/mapmaking/noise.py:705-708), batched over every mode of every
- * TOD.  Exact for any n: rows of about 1400 to 2^19 samples run as a
- * Toeplitz product and its reversal through one real FFT of L >= 2n-1 points
- * (L = 2^12 q1, q1 from a fixed list), others as one circular convolution
- * through L = 2^q >= 3(n-1)+1 points.  FP32 lengths are chosen and reported
- * as classes P1, 5-smooth in [2, 256] with 2^12 P1 >= 3(n-1)+1 (by default
- * the smallest); q1 follows from n, or from a longer class.
+ * TOD.  Computed as one circular convolution per row through a real FFT of
+ * L >= 3(n-1)+1 points (exact for any n): L = 2^11 P1 with P1 5-smooth in
+ * [2, 256] on the FP32 path (by default the smallest such L), else
+ * L = 2^q.
  * desc (host): 6 int64 per segment (TOD): rows, n, in_off, in_stride,
  *   out_off, out_stride (element offsets into the exec in/out arrays).
  * elem_bytes: 4 (FP32 transform) or 8 (FP64 transform).
  * The plan owns its spectra (allocated by mk_filt_plan_set_weights; a plan
  * whose segments all borrow spectra holds none) and a work buffer of
- * rows*(P+1) complex values (P = L/2), allocated by the first call that
- * needs it (so capture a graph only after one eager exec) and freed by
+ * rows*P complex values, allocated by the first call that needs it (so
+ * capture a graph only after one eager exec) and freed by
  * mk_filt_plan_release_work, or supplied by the caller
  * (mk_filt_plan_set_work). */
 typedef struct mk_filt_plan mk_filt_plan;
 int mk_filt_plan_create(int nseg, const int64_t *desc, int elem_bytes,
                         mk_filt_plan **plan);
-/* As mk_filt_plan_create, with the length class P1 of every segment chosen
+/* As mk_filt_plan_create, with the column length P1 of every segment chosen
  * by the caller (an autotuner; the FFTW-wisdom counterpart of
  * minkasi/tools/fft.py:347-384): p1[i] = 0 keeps the default, otherwise it
  * must be one of the FP32 hot lengths (mk_filt_hot_p1) with
@@ -339,7 +335,7 @@ int mk_filt_plan_create(int nseg, const int64_t *desc, int elem_bytes,
  * borrowed must agree on P1. */
 int mk_filt_plan_create_p1(int nseg, const int64_t *desc, int elem_bytes,
                            const int32_t *p1, mk_filt_plan **plan);
-/* Writes up to cap length classes (ascending) to out (may be NULL) and
+/* Writes up to cap hot column lengths (ascending) to out (may be NULL) and
  * returns how many there are. */
 int mk_filt_hot_p1(int32_t *out, int cap);
 /* wdct: device FP64, rows of C W (the DCT-I of each row of mywt), laid out
@@ -360,7 +356,7 @@ int mk_filt_plan_exec_f32(const mk_filt_plan *plan, const float *in,
 /* Frees the work buffer (synchronises the stream first); a caller's buffer
  * (mk_filt_plan_set_work) is only detached. */
 int mk_filt_plan_release_work(mk_filt_plan *plan, void *stream);
-/* Bytes of work buffer the plan needs (at most rows * (P + 1) complex values). */
+/* Bytes of work buffer the plan needs (rows * P complex values). */
 int mk_filt_plan_work_bytes(const mk_filt_plan *plan, int64_t *bytes);
 /* Makes the plan use the caller's device buffer (>= mk_filt_plan_work_bytes,
  * 16-byte aligned) as its work buffer instead of one of its own; NULL
@@ -376,9 +372,7 @@ int mk_filt_plan_exec_f64(const mk_filt_plan *plan, const double *in,
 /* info[0..7] = nseg, K1/K3 items, K2 items, work bytes, spectrum bytes,
  * elem_bytes, LDS bytes K1/K3, LDS bytes K2. */
 int mk_filt_plan_info(const mk_filt_plan *plan, int64_t *info);
-/* geom[4*i..4*i+3] = P1, P2, columns per item, P1 P2 of segment i; for rows
- * longer than 2^11 * 2/3 samples P1 is the length class (P2 = 2^11), of which
- * the transform itself needs about two thirds. */
+/* geom[4*i..4*i+3] = P1, P2, columns per item, P of segment i. */
 int mk_filt_plan_geometry(const mk_filt_plan *plan, int64_t *geom);
 int mk_filt_plan_destroy(mk_filt_plan *plan);
 

@@ -6,55 +6,69 @@
 // scipy.fft.dct type 1, minkasi/tools/py_fft.py:239) and W = mywt.  With
 // m = n-1 and N = 2m, C W C y = (even extension of y) circularly convolved
 // (period N) with h = C W (because C C = N I).  The engine evaluates that
-// circular convolution exactly through real FFTs, for any n (no Bluestein,
-// no smooth-length requirement), and fuses the forward transform, the weight
-// multiply and the inverse transform.  Two forms:
-//
-//  2^11-row path (FP32 and FP64 rows of about 1400 to 2^19 samples;
-//  fft_cols.h, fft_rows.hip).  With the end samples halved, the output is
-//  sum_j y_j [h(k-j) + h(k+j)], a Toeplitz product plus one with a kernel
-//  reversed about m/2 (h(k+j) = h(k - (m-j) + m)): as spectra
-//  H Y + G phi conj(Y) with Y one real transform of L >= 2m+1 points, H and
-//  G the real spectra of h(|t|) and h(m-|t|), |t| <= m, and phi the phase of
-//  the reversal's centre.  L = 2^12 q1, q1 the smallest of 41 counts that
-//  split into two radices up to 16.
-//
-//  General path (shorter and longer rows).  The even extension on [-m, 2m]
-//  through L >= 3m+1 points with one real spectrum; the outputs needed are
-//  the window [m, 2m]; L a power of two.
+// circular convolution exactly as a linear one through a real FFT of
+// L >= 3m+1 points: the input is the even periodic extension z' on
+// [-m, 2m], the kernel is h placed symmetrically (so its spectrum B is real
+// and even), and the outputs needed are the window [m, 2m].  This works for
+// any n (no Bluestein, no smooth-length requirement) and fuses the forward
+// transform, the weight multiply and the inverse transform.  L is the
+// smallest 4096 P1 >= 3m+1 with P1 5-smooth (<= 256) on the FP32 hot path,
+// else the next power of two.
 //
 // Stand-alone DCT-I (fft_r2r, minkasi/tools/fft.py:290-344) uses Bluestein's
 // chirp-z algorithm (Bluestein 1970; Rabiner, Schafer & Rader 1969) on the
-// same engines: Y_k = Re(chi_k sum_j c_j x_j chi_j conj(chi_{k-j})) with
+// same engine: Y_k = Re(chi_k sum_j c_j x_j chi_j conj(chi_{k-j})) with
 // chi_j = exp(-i pi j^2 / N), c_j = 1 at j = 0, m and 2 otherwise, the
-// convolution evaluated with a complex FFT of P >= 2m+1 points (FP64: 2^11 q1,
-// else a power of two).
+// convolution evaluated with a complex FFT of P = 2^q >= 2m+1 points.
 //
-// General path's four-step layout (P = P1*P2 complex points, j = P2*j1 + j2,
-// k = k1 + P1*k2):
+// Four-step layout (P = P1*P2 complex points, j = P2*j1 + j2, k = k1 + P1*k2):
 //   K1: column FFTs of length P1 (one workgroup = cw adjacent columns, so
 //       global reads are contiguous runs), twiddle w_P^(j2*k1), store T[k1][j2].
 //   K2: row FFTs of length P2 (rows k1 and P1-k1 together, which is where the
 //       real-FFT unpacking partner C_(P-k) lives), pointwise spectral work,
 //       inverse row FFTs, conjugate twiddle, store back.
 //   K3: inverse column FFTs of length P1, 1/P scale, write the wanted outputs.
-// Every LDS sub-FFT is a Stockham pass sequence (radix 8, then 4 or 2) with a
-// stage-ordered twiddle table.
+// Every LDS sub-FFT is a Stockham pass sequence (radix 8, then 4 or 2; radix
+// 3 and 5 for mixed column lengths) with a stage-ordered twiddle table.
 // Each launch covers every row of every segment (TOD) in the batch through
 // a work list.
-#include "fft_engine.h"
+#include "common.h"
 
 #include <algorithm>
 #include <cstdlib>
 #include <mutex>
 #include <vector>
 
-using namespace mkfft;
-
 namespace {
 
-// exp(-i*pi*num*inv_den) with 1/inv_den a power of two and num < 2^24, so
-// -num * inv_den is exact in T.
+template <typename T>
+struct cx {
+  T re, im;
+};
+template <typename T>
+__device__ __forceinline__ cx<T> cadd(cx<T> a, cx<T> b) { return {a.re + b.re, a.im + b.im}; }
+template <typename T>
+__device__ __forceinline__ cx<T> csub(cx<T> a, cx<T> b) { return {a.re - b.re, a.im - b.im}; }
+template <typename T>
+__device__ __forceinline__ cx<T> cmul(cx<T> a, cx<T> b) {
+  return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
+}
+template <typename T>
+__device__ __forceinline__ cx<T> cconj(cx<T> a) { return {a.re, -a.im}; }
+template <typename T>
+__device__ __forceinline__ cx<T> cscale(cx<T> a, T s) { return {a.re * s, a.im * s}; }
+
+__device__ __forceinline__ void sincospi_t(float x, float* s, float* c) { sincospif(x, s, c); }
+__device__ __forceinline__ void sincospi_t(double x, double* s, double* c) { sincospi(x, s, c); }
+
+// exp(-i*pi*num/den) for integers 0 <= num < 2*den.  expmi2 requires den a
+// power of two and num < 2^24, so -num * (1/den) is exact in T.
+template <typename T>
+__device__ __forceinline__ cx<T> expmi(int64_t num, int64_t den) {
+  T s, c;
+  sincospi_t((T)(-(double)num / (double)den), &s, &c);
+  return {c, s};
+}
 template <typename T>
 __device__ __forceinline__ cx<T> expmi2(int64_t num, T inv_den) {
   T s, c;
@@ -78,6 +92,46 @@ constexpr __host__ __device__ __forceinline__ int pad8(int e) { return e + (e >>
 // Odd, so that rows read in parallel fall in different banks (for a power of
 // two len this is len + len/16 + 1).
 constexpr __host__ __device__ __forceinline__ int row_stride(int len) { return (len + (len >> MK_FFT_PAD_SHIFT)) | 1; }
+
+// In-register DFTs (natural order in and out).
+template <typename T, bool INV>
+__device__ __forceinline__ void dft2(cx<T>* v) {
+  cx<T> a = v[0], b = v[1];
+  v[0] = cadd(a, b);
+  v[1] = csub(a, b);
+}
+template <typename T, bool INV>
+__device__ __forceinline__ void dft4(cx<T>& a0, cx<T>& a1, cx<T>& a2, cx<T>& a3) {
+  cx<T> b0 = cadd(a0, a2), b1 = csub(a0, a2), b2 = cadd(a1, a3), d = csub(a1, a3);
+  cx<T> b3 = INV ? cx<T>{-d.im, d.re} : cx<T>{d.im, -d.re};  // (+/-i) * d
+  a0 = cadd(b0, b2);
+  a2 = csub(b0, b2);
+  a1 = cadd(b1, b3);
+  a3 = csub(b1, b3);
+}
+template <typename T, bool INV>
+__device__ __forceinline__ void dft4v(cx<T>* v) { dft4<T, INV>(v[0], v[1], v[2], v[3]); }
+template <typename T, bool INV>
+__device__ __forceinline__ void dft8(cx<T>* v) {
+  const T c = T(0.70710678118654752440);
+  cx<T> e0 = v[0], e1 = v[2], e2 = v[4], e3 = v[6];
+  cx<T> o0 = v[1], o1 = v[3], o2 = v[5], o3 = v[7];
+  dft4<T, INV>(e0, e1, e2, e3);
+  dft4<T, INV>(o0, o1, o2, o3);
+  if (!INV) {
+    o1 = {c * (o1.re + o1.im), c * (o1.im - o1.re)};   // * exp(-i pi/4)
+    o2 = {o2.im, -o2.re};                               // * -i
+    o3 = {c * (o3.im - o3.re), -c * (o3.re + o3.im)};  // * exp(-3i pi/4)
+  } else {
+    o1 = {c * (o1.re - o1.im), c * (o1.re + o1.im)};   // * exp(i pi/4)
+    o2 = {-o2.im, o2.re};                               // * i
+    o3 = {-c * (o3.re + o3.im), c * (o3.re - o3.im)};  // * exp(3i pi/4)
+  }
+  v[0] = cadd(e0, o0); v[4] = csub(e0, o0);
+  v[1] = cadd(e1, o1); v[5] = csub(e1, o1);
+  v[2] = cadd(e2, o2); v[6] = csub(e2, o2);
+  v[3] = cadd(e3, o3); v[7] = csub(e3, o3);
+}
 
 // One radix-R Stockham stage over nrows padded rows of length 2^l2len.
 // Every thread loads all of its butterflies' inputs, the workgroup
@@ -171,6 +225,160 @@ __device__ void fill_stage_table(cx<T>* tab, int l2len) {
 template <typename T>
 __device__ __forceinline__ cx<T> twiddle_P(int64_t a, T invP) { return expmi2<T>(2 * a, invP); }
 
+// ---- Mixed radix (2, 3, 5) transform lengths ---------------------------------
+// Radix of the next stage of an N-point Stockham FFT when rem = N / Ns points
+// per sub-transform remain to be combined: the power-of-two part first (8
+// while 8 divides rem, then one 4 or 2; for N = 2^q this is the stage_lr
+// sequence), then 3s, then 5s.  Stage tables are laid out in this order.
+constexpr __host__ __device__ int next_radix(int rem) {
+  return (rem & 1) == 0 ? ((rem & 7) == 0 ? 8 : ((rem & 3) == 0 ? 4 : 2)) : (rem % 3 == 0 ? 3 : 5);
+}
+
+template <typename T, bool INV>
+__device__ __forceinline__ void dft3(cx<T>* v) {
+  const T h = T(0.86602540378443864676);  // sin(2 pi / 3)
+  cx<T> a = cadd(v[1], v[2]), d = csub(v[1], v[2]);
+  cx<T> t = {v[0].re - T(0.5) * a.re, v[0].im - T(0.5) * a.im};
+  cx<T> u = INV ? cx<T>{-h * d.im, h * d.re} : cx<T>{h * d.im, -h * d.re};  // (+/-i) sin(2pi/3) d
+  v[0] = cadd(v[0], a);
+  v[1] = cadd(t, u);
+  v[2] = csub(t, u);
+}
+template <typename T, bool INV>
+__device__ __forceinline__ void dft5(cx<T>* v) {
+  const T c1 = T(0.30901699437494742410), c2 = T(-0.80901699437494742410);  // cos(2pi/5), cos(4pi/5)
+  const T s1 = T(0.95105651629515357212), s2 = T(0.58778525229247312917);   // sin(2pi/5), sin(4pi/5)
+  cx<T> a1 = cadd(v[1], v[4]), b1 = csub(v[1], v[4]), a2 = cadd(v[2], v[3]), b2 = csub(v[2], v[3]);
+  cx<T> t1 = {v[0].re + c1 * a1.re + c2 * a2.re, v[0].im + c1 * a1.im + c2 * a2.im};
+  cx<T> t2 = {v[0].re + c2 * a1.re + c1 * a2.re, v[0].im + c2 * a1.im + c1 * a2.im};
+  cx<T> u1 = {s1 * b1.re + s2 * b2.re, s1 * b1.im + s2 * b2.im};
+  cx<T> u2 = {s2 * b1.re - s1 * b2.re, s2 * b1.im - s1 * b2.im};
+  // forward: y1 = t1 - i u1, y4 = t1 + i u1, y2 = t2 - i u2, y3 = t2 + i u2
+  cx<T> iu1 = INV ? cx<T>{-u1.im, u1.re} : cx<T>{u1.im, -u1.re};
+  cx<T> iu2 = INV ? cx<T>{-u2.im, u2.re} : cx<T>{u2.im, -u2.re};
+  v[0] = cadd(v[0], cadd(a1, a2));
+  v[1] = cadd(t1, iu1);
+  v[4] = csub(t1, iu1);
+  v[2] = cadd(t2, iu2);
+  v[3] = csub(t2, iu2);
+}
+template <typename T, bool INV, int R>
+__device__ __forceinline__ void dft_r(cx<T>* v) {
+  if constexpr (R == 8) dft8<T, INV>(v);
+  else if constexpr (R == 4) dft4v<T, INV>(v);
+  else if constexpr (R == 2) dft2<T, INV>(v);
+  else if constexpr (R == 3) dft3<T, INV>(v);
+  else dft5<T, INV>(v);
+}
+
+// One radix-R stage of an N-point mixed-radix Stockham FFT over nrows padded
+// rows (the runtime counterpart of fft_stage): butterfly j of a row reads
+// j + r N/R, twiddles by tw[(r-1) Ns + k] (k = j mod Ns) and writes
+// (j / Ns) Ns R + k + r Ns.
+template <typename T, bool INV, int R>
+__device__ __forceinline__ void fft_stage_mx(cx<T>* buf, const cx<T>* tw, int N, int nrows, int rs, int Ns) {
+  constexpr int NB = (kMaxWG / R + kThreads - 1) / kThreads;
+  const int q = N / R, nbf = nrows * q;
+  cx<T> v[NB][R];
+#pragma unroll
+  for (int u = 0; u < NB; u++) {
+    const int bf = threadIdx.x + u * kThreads;
+    if (bf < nbf) {
+      const int row = bf / q, j = bf - row * q, k = j % Ns;
+      const cx<T>* base = buf + row * rs;
+#pragma unroll
+      for (int r = 0; r < R; r++) v[u][r] = base[pad8(j + r * q)];
+      if (Ns > 1) {
+#pragma unroll
+        for (int r = 1; r < R; r++) {
+          cx<T> w = tw[(r - 1) * Ns + k];
+          if (INV) w = cconj(w);
+          v[u][r] = cmul(v[u][r], w);
+        }
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < NB; u++) {
+    const int bf = threadIdx.x + u * kThreads;
+    if (bf < nbf) {
+      const int row = bf / q, j = bf - row * q, k = j % Ns;
+      dft_r<T, INV, R>(v[u]);
+      cx<T>* base = buf + row * rs;
+      const int idx = (j / Ns) * Ns * R + k;
+#pragma unroll
+      for (int r = 0; r < R; r++) base[pad8(idx + r * Ns)] = v[u][r];
+    }
+  }
+  __syncthreads();
+}
+
+// In-place N-point FFT (N 5-smooth) of nrows padded rows, nrows * N <= kMaxWG;
+// tw = fill_stage_table_mx table.
+template <typename T, bool INV>
+__device__ void lds_fft_mx(cx<T>* buf, const cx<T>* tw, int N, int nrows, int rs) {
+  int Ns = 1, off = 0;
+  while (Ns < N) {
+    const int R = next_radix(N / Ns);
+    switch (R) {
+      case 8: fft_stage_mx<T, INV, 8>(buf, tw + off, N, nrows, rs, Ns); break;
+      case 4: fft_stage_mx<T, INV, 4>(buf, tw + off, N, nrows, rs, Ns); break;
+      case 2: fft_stage_mx<T, INV, 2>(buf, tw + off, N, nrows, rs, Ns); break;
+      case 3: fft_stage_mx<T, INV, 3>(buf, tw + off, N, nrows, rs, Ns); break;
+      default: fft_stage_mx<T, INV, 5>(buf, tw + off, N, nrows, rs, Ns); break;
+    }
+    off += (R - 1) * Ns;
+    Ns *= R;
+  }
+}
+
+// Stage table of an N-point mixed-radix FFT (next_radix order): entry
+// (r-1) Ns + k of a stage is exp(-2 pi i k r / (R Ns)); N - 1 entries.
+template <typename T>
+__device__ void fill_stage_table_mx(cx<T>* tab, int N) {
+  int Ns = 1, off = 0;
+  while (Ns < N) {
+    const int R = next_radix(N / Ns), cnt = (R - 1) * Ns;
+    for (int e = threadIdx.x; e < cnt; e += blockDim.x) {
+      const int r = e / Ns + 1, k = e - (r - 1) * Ns;
+      tab[off + e] = expmi<T>(2 * (int64_t)k * r, (int64_t)R * Ns);
+    }
+    off += cnt;
+    Ns *= R;
+  }
+}
+
+// exp(-2 pi i a / P) for 0 <= a < P and any P (FP64 argument reduction).
+template <typename T>
+__device__ __forceinline__ cx<T> twiddle_any(int64_t a, int64_t P) { return expmi<T>(2 * a, P); }
+
+// Segment: `rows` rows sharing one length n and one plan.
+struct Seg {
+  int64_t in_off, in_stride;    // input rows (elements of the input type)
+  int64_t out_off, out_stride;  // output rows
+  int64_t t_off, t_stride;      // T buffer rows (complex)
+  int64_t s_off, s_stride;      // spectrum rows (filter: P+1 reals; Bluestein: P complex, stride 0)
+  void* s_ptr;                  // device address of this segment's spectrum rows (set at upload)
+  void* tw_ptr;                 // hot K2: fine/coarse twiddle tables of this P (set at create)
+  int32_t rows, n, l1, l2, cw, flags;  // l1 = log2(P1), or -1 when P1 is not a power of two
+  int64_t base1, base2, base3;  // first global item of K1, K2, K3
+  int32_t per1, per2;           // items per row for K1/K3, K2
+  int32_t r2, p1;               // k1 values per K2 item; column length P1 (2^a 3^b 5^c)
+};
+
+enum Mode { kFilter = 0, kFSpec = 1, kBlue = 2, kBSpec = 3 };
+
+__device__ inline int find_seg(const Seg* segs, int nseg, int64_t g, int which) {
+  int lo = 0, hi = nseg - 1;
+  while (lo < hi) {
+    int mid = (lo + hi + 1) >> 1;
+    int64_t b = which == 1 ? segs[mid].base1 : (which == 2 ? segs[mid].base2 : segs[mid].base3);
+    if (b <= g) lo = mid; else hi = mid - 1;
+  }
+  return lo;
+}
+
 // ---- K1: column FFTs -------------------------------------------------------
 // LDS: cw padded rows of length P1 (one per matrix column j2), then the P1
 // twiddle table and the P2 table exp(-2 pi i j/P) for the four-step twiddle.
@@ -183,6 +391,10 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 1) k1_kernel(co
   const int64_t local = (int64_t)blockIdx.x - sg.base1;
   const int row = (int)(local / sg.per1), jb = (int)(local % sg.per1);
   const int l1 = sg.l1, l2 = sg.l2, P1 = sg.p1, P2 = 1 << l2, cw = sg.cw;
+  // Mixed-radix column lengths reach this kernel only in the spectrum pass
+  // (the filter runs them on the hot path), so only that mode carries the
+  // mixed-radix code.
+  const bool pow2 = MODE != kFSpec || l1 >= 0;
   const int lcw = 31 - __clz(cw);
   const int rs = row_stride(P1);
   const int64_t P = (int64_t)P1 * P2;
@@ -191,7 +403,8 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 1) k1_kernel(co
   cx<T>* tw = buf + cw * rs;                          // [P1] stage table
   const TIn* x = in + sg.in_off + (int64_t)row * sg.in_stride;
   const int j2_0 = jb * cw;
-  fill_stage_table<T>(tw, l1);
+  if (pow2) fill_stage_table<T>(tw, l1);
+  else if constexpr (MODE == kFSpec) fill_stage_table_mx<T>(tw, P1);
   constexpr int UNR = 8;  // loads in flight per thread
   if (MODE == kFilter || MODE == kFSpec) {
     // real input packed two per complex point: a_(2j), a_(2j+1)
@@ -250,14 +463,15 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 1) k1_kernel(co
     }
   }
   __syncthreads();
-  lds_fft<T, false>(buf, tw, l1, cw, rs);
+  if (pow2) lds_fft<T, false>(buf, tw, l1, cw, rs);
+  else if constexpr (MODE == kFSpec) lds_fft_mx<T, false>(buf, tw, P1, cw, rs);
   cx<T>* trow = tbuf + sg.t_off + (int64_t)row * sg.t_stride;
   const T invP = T(1) / (T)P;
   for (int idx = threadIdx.x; idx < P1 * cw; idx += kThreads) {
     int k1 = idx >> lcw, c = idx & (cw - 1);
     int64_t j2 = j2_0 + c;
     int64_t a = (j2 * k1) % P;
-    cx<T> v = cmul(buf[c * rs + pad8(k1)], twiddle_P<T>(a, invP));
+    cx<T> v = cmul(buf[c * rs + pad8(k1)], pow2 ? twiddle_P<T>(a, invP) : twiddle_any<T>(a, P));
     trow[(int64_t)k1 * P2 + j2] = v;
   }
 }
@@ -281,6 +495,7 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 1) k2_kernel(co
   const int64_t local = (int64_t)blockIdx.x - sg.base2;
   const int row = (int)(local / sg.per2), grp = (int)(local % sg.per2);
   const int l2 = sg.l2, P1 = sg.p1, P2 = 1 << l2;
+  const bool pow2 = sg.l1 >= 0;
   const int rs = row_stride(P2);
   const int64_t P = (int64_t)P1 * P2;
   const bool real_mode = (MODE == kFilter || MODE == kFSpec);
@@ -368,7 +583,7 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 1) k2_kernel(co
       cx<T> E = cscale(cadd(C, cconj(Cq)), T(0.5));
       cx<T> Dd = csub(C, cconj(Cq));
       cx<T> O = {Dd.im * T(0.5), -Dd.re * T(0.5)};
-      cx<T> w = expmi2<T>(k, invP);  // w_L^k; w_L^(P-k) = -conj(w)
+      cx<T> w = pow2 ? expmi2<T>(k, invP) : expmi<T>(k, P);  // w_L^k; w_L^(P-k) = -conj(w)
       cx<T> A = cadd(E, cmul(w, O));
       cx<T> Aq = csub(cconj(E), cmul(cconj(w), cconj(O)));
       int pk1 = slot_k1[pidx >> l2], pk2 = pidx & (P2 - 1);
@@ -407,26 +622,436 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 1) k2_kernel(co
     int sl = idx >> l2, j2 = idx & (P2 - 1);
     int kk1 = slot_k1[sl];
     int64_t a = ((int64_t)j2 * kk1) % P;
-    trow[(int64_t)kk1 * P2 + j2] = cmul(at(idx), cconj(twiddle_P<T>(a, invP2)));
+    trow[(int64_t)kk1 * P2 + j2] = cmul(at(idx), cconj(pow2 ? twiddle_P<T>(a, invP2) : twiddle_any<T>(a, P)));
   }
 }
 
-// ---- Length classes of the 2^11-point-row engine ----------------------------
-// A row of n samples belongs to the class P1, the smallest 5-smooth number in
-// [2, 256] with 2^11 P1 >= 1.5 (n-1) + 1 (or a larger one of the caller's
-// choice): the unit in which the autotuner compares and fixes transform
-// lengths, and what mk_filt_plan_geometry reports.  The transform itself
-// needs 2^11 q1 >= n only, two thirds of the class's length.
-constexpr int kHotL2 = kRowL2;
-constexpr int kHotP2 = kRowLen;
+// ---- K2, FP32 filter hot path: rows of 2^11 points --------------------------
+// Every workgroup holds exactly two rows: k1 and its partner P1-k1, or, for
+// the first workgroup of a mode, the self-paired rows k1 = 0 and (even P1)
+// P1/2; with odd P1 the second slot of that workgroup is idle.
+// Stage and four-step twiddles come from tables built once per plan in FP64
+// (no transcendental in the loop); the stage shapes are compile-time, so the
+// LDS addresses fold into instruction offsets.  Each thread owns four
+// (k, P-k) pairs of the spectral step (five for thread 0 of workgroup 0).
+constexpr int kHotL2 = 11;
+constexpr int kHotP2 = 1 << kHotL2;
+constexpr int kHotRS = row_stride(kHotP2);
+constexpr int kHotMaxL1 = 8;                  // P1 <= 256
+constexpr int kFineBits = 10;                 // fine table: 1024 entries of w_2P
+// X rows + fine/coarse tables; the stage twiddles are read from the global
+// table (16 KB, L1-resident), which keeps three workgroups per CU.
+constexpr int kHotLds = (2 * kHotRS + (1 << kFineBits) + (4 << kHotMaxL1)) * 8;
+
+// Compile-time Stockham stage over NROWS padded rows (stride RS) of 2^L2LEN
+// points; NROWS * 2^L2LEN = kMaxWG.
+template <bool INV, int LR, int L2LEN, int LNS, int NROWS, int RS>
+__device__ __forceinline__ void ct_stage(cx<float>* buf, const cx<float>* tw) {
+  constexpr int R = 1 << LR;
+  constexpr int NB = (NROWS << L2LEN) / R / kThreads;
+  static_assert(NB >= 1 && NB * R * kThreads == (NROWS << L2LEN), "stage does not tile the workgroup");
+  constexpr int LQ = L2LEN - LR, Q = 1 << LQ, NS = 1 << LNS;
+  cx<float> v[NB][R];
+#pragma unroll
+  for (int u = 0; u < NB; u++) {
+    const int bf = threadIdx.x + u * kThreads;
+    const int row = bf >> LQ, j = bf & (Q - 1), k = j & (NS - 1);
+    const cx<float>* base = buf + row * RS;
+#pragma unroll
+    for (int r = 0; r < R; r++) v[u][r] = base[pad8(j + r * Q)];
+    if (LNS > 0) {
+#pragma unroll
+      for (int r = 1; r < R; r++) {
+        cx<float> w = tw[(r - 1) * NS + k];
+        if (INV) w = cconj(w);
+        v[u][r] = cmul(v[u][r], w);
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < NB; u++) {
+    const int bf = threadIdx.x + u * kThreads;
+    const int row = bf >> LQ, j = bf & (Q - 1), k = j & (NS - 1);
+    if (LR == 3) dft8<float, INV>(v[u]);
+    else if (LR == 2) dft4v<float, INV>(v[u]);
+    else dft2<float, INV>(v[u]);
+    cx<float>* base = buf + row * RS;
+    const int idx = ((j >> LNS) << (LNS + LR)) + k;
+#pragma unroll
+    for (int r = 0; r < R; r++) base[pad8(idx + r * NS)] = v[u][r];
+  }
+  __syncthreads();
+}
+
+// FFT of NROWS rows of 2^L2LEN points, stages of radix 8 then 4 or 2; st is
+// the stage-ordered table (fill_stage_table order).
+template <bool INV, int L2LEN, int NROWS, int RS, int LNS = 0, int OFF = 0>
+__device__ __forceinline__ void ct_fft(cx<float>* buf, const cx<float>* st) {
+  if constexpr (LNS < L2LEN) {
+    constexpr int LR = (L2LEN - LNS) >= 3 ? 3 : (L2LEN - LNS);
+    ct_stage<INV, LR, L2LEN, LNS, NROWS, RS>(buf, st + OFF);
+    ct_fft<INV, L2LEN, NROWS, RS, LNS + LR, OFF + ((1 << LR) - 1) * (1 << LNS)>(buf, st);
+  }
+}
+
+__device__ __forceinline__ cx<float> tw2P(const cx<float>* F, const cx<float>* C, int k) {
+  return cmul(F[k & ((1 << kFineBits) - 1)], C[k >> kFineBits]);  // w_2P^k
+}
+
+__global__ void __launch_bounds__(kThreads, 4) k2_hot_kernel(const Seg* __restrict__ segs, int nseg,
+                                                              cx<float>* __restrict__ tbuf,
+                                                              const cx<float>* __restrict__ stab_g) {
+  extern __shared__ unsigned char smem_raw[];
+  const int s = find_seg(segs, nseg, blockIdx.x, 2);
+  const Seg sg = segs[s];
+  const int local = (int)((int64_t)blockIdx.x - sg.base2);
+  const int row = local / sg.per2, g = local - row * sg.per2;
+  const int P1 = sg.p1;
+  const int P = P1 << kHotL2;
+  const bool single = g == 0 && (P1 & 1);  // odd P1: column 0 is the only self-paired one
+  const int kA = g == 0 ? 0 : g, kB = g == 0 ? (single ? 0 : P1 / 2) : P1 - g;
+  cx<float>* X = reinterpret_cast<cx<float>*>(smem_raw);  // [2][kHotRS]
+  cx<float>* F = X + 2 * kHotRS;                           // [1024] w_2P^l
+  cx<float>* Ct = F + (1 << kFineBits);                    // [4 P1] w_2P^(1024 h)
+  const cx<float>* st = stab_g;                            // stage table (global)
+  const cx<float>* twF = reinterpret_cast<const cx<float>*>(sg.tw_ptr);
+  const int nC = 4 * P1;
+  for (int e = threadIdx.x; e < (1 << kFineBits); e += kThreads) F[e] = twF[e];
+  for (int e = threadIdx.x; e < nC; e += kThreads) Ct[e] = twF[(1 << kFineBits) + e];
+  cx<float>* trow = tbuf + sg.t_off + (int64_t)row * sg.t_stride;
+  const float* srow = reinterpret_cast<const float*>(sg.s_ptr) + (int64_t)row * sg.s_stride;
+  {
+    cx<float> va[4], vb[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int k2 = threadIdx.x + u * kThreads;
+      va[u] = trow[kA * kHotP2 + k2];
+      vb[u] = trow[kB * kHotP2 + k2];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int k2 = threadIdx.x + u * kThreads;
+      X[pad8(k2)] = va[u];
+      X[kHotRS + pad8(k2)] = vb[u];
+    }
+  }
+  // this thread's pairs: (slot, k2) <-> (slot_q, k2q)
+  constexpr int NPAIR = 5;
+  int p_sl[NPAIR], p_k2[NPAIR], p_slq[NPAIR], p_k2q[NPAIR];
+  float bb[NPAIR], bq[NPAIR];
+  float bP = 0.f;
+#pragma unroll
+  for (int u = 0; u < NPAIR; u++) {
+    const int pl = threadIdx.x + u * kThreads;
+    int sl = -1, k2 = 0, slq = 0, k2q = 0;
+    if (g != 0) {
+      if (pl < kHotP2) { sl = 0; k2 = pl; slq = 1; k2q = kHotP2 - 1 - pl; }
+    } else if (pl <= kHotP2 / 2) {
+      sl = 0; k2 = pl; slq = 0; k2q = (kHotP2 - pl) & (kHotP2 - 1);
+    } else if (!single && pl < kHotP2 + 1) {
+      sl = 1; k2 = pl - (kHotP2 / 2 + 1); slq = 1; k2q = kHotP2 - 1 - k2;
+    }
+    p_sl[u] = sl; p_k2[u] = k2; p_slq[u] = slq; p_k2q[u] = k2q;
+    bb[u] = bq[u] = 0.f;
+    if (sl >= 0) {
+      bb[u] = srow[(sl ? kB : kA) * kHotP2 + k2];
+      bq[u] = srow[(slq ? kB : kA) * kHotP2 + k2q];
+    }
+  }
+  if (g == 0 && threadIdx.x == 0) bP = srow[P];
+  __syncthreads();
+  // twiddles factor along k2 = tid + 512 u:  w_2P^(k1 + P1 k2) =
+  // w_2P^k1 * w_4096^tid * w_8^u, and w_P^(k1 j2) = w_P^(k1 tid) * (w_P^(512 k1))^u
+  cx<float> w4096t;
+  sincospif(-(float)threadIdx.x * (1.f / 2048.f), &w4096t.im, &w4096t.re);
+  const cx<float> wkA = tw2P(F, Ct, kA), wkB = tw2P(F, Ct, kB);
+  ct_fft<false, kHotL2, 2, kHotRS>(X, st);
+#pragma unroll
+  for (int u = 0; u < NPAIR; u++) {
+    const int sl = p_sl[u];
+    if (sl < 0) continue;
+    const int k2 = p_k2[u], slq = p_slq[u], k2q = p_k2q[u];
+    const int kk1 = sl ? kB : kA;
+    const int idx = sl * kHotRS + pad8(k2), pidx = slq * kHotRS + pad8(k2q);
+    const int k = kk1 + P1 * k2;
+    cx<float> C = X[idx], Cq = X[pidx];
+    cx<float> E = cscale(cadd(C, cconj(Cq)), 0.5f);
+    cx<float> Dd = csub(C, cconj(Cq));
+    cx<float> O = {Dd.im * 0.5f, -Dd.re * 0.5f};
+    cx<float> w;
+    if (k2 == (int)threadIdx.x + u * kThreads) {  // every pair but those of the row k1 = P1/2 of workgroup 0
+      constexpr float c8 = 0.70710678118654752440f;
+      const cx<float> w8[4] = {{1.f, 0.f}, {c8, -c8}, {0.f, -1.f}, {-c8, -c8}};
+      w = cmul(cmul(sl ? wkB : wkA, w4096t), w8[u & 3]);
+    } else {
+      w = tw2P(F, Ct, k);
+    }
+    cx<float> A = cadd(E, cmul(w, O));
+    cx<float> Aq = csub(cconj(E), cmul(cconj(w), cconj(O)));
+    cx<float> Y = cscale(A, bb[u]), Yq = cscale(Aq, bq[u]);
+    if (k == 0) {
+      const float yP = (E.re - O.re) * bP;
+      cx<float> Ep = {0.5f * (Y.re + yP), 0.5f * Y.im};
+      cx<float> Op = {0.5f * (Y.re - yP), 0.5f * Y.im};
+      X[idx] = {Ep.re - Op.im, Ep.im + Op.re};
+      continue;
+    }
+    cx<float> Ep = cscale(cadd(Y, cconj(Yq)), 0.5f);
+    cx<float> Op = cmul(cscale(csub(Y, cconj(Yq)), 0.5f), cconj(w));
+    cx<float> Eq = cscale(cadd(Yq, cconj(Y)), 0.5f);
+    cx<float> Oq = cmul(cscale(csub(Yq, cconj(Y)), 0.5f), cx<float>{-w.re, -w.im});
+    X[idx] = {Ep.re - Op.im, Ep.im + Op.re};
+    if (pidx != idx) X[pidx] = {Eq.re - Oq.im, Eq.im + Oq.re};
+  }
+  __syncthreads();
+  ct_fft<true, kHotL2, 2, kHotRS>(X, st);
+  // kA, kB < 256 and tid < 512, so the products fit in 32 bits
+  const uint32_t uP = (uint32_t)P;
+  cx<float> tA = tw2P(F, Ct, 2 * (int)(((uint32_t)kA * threadIdx.x) % uP));
+  cx<float> tB = tw2P(F, Ct, 2 * (int)(((uint32_t)kB * threadIdx.x) % uP));
+  const cx<float> sA = tw2P(F, Ct, 2 * (int)(((uint32_t)kA * kThreads) % uP));
+  const cx<float> sB = tw2P(F, Ct, 2 * (int)(((uint32_t)kB * kThreads) % uP));
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    const int j2 = threadIdx.x + u * kThreads;
+    trow[kA * kHotP2 + j2] = cmul(X[pad8(j2)], cconj(tA));
+    if (!single) trow[kB * kHotP2 + j2] = cmul(X[kHotRS + pad8(j2)], cconj(tB));
+    tA = cmul(tA, sA);
+    tB = cmul(tB, sB);
+  }
+}
+
+// ---- K1 / K3, FP32 filter hot path: columns of P1 = 2^a 3^b 5^c (rows of 2^11)
+// One launch per column length; CW adjacent columns per workgroup (the
+// largest power of two with CW P1 <= 4096, but at least 32), so global reads
+// and writes are runs of CW points.  The LDS tile is column-major: point j
+// of column c at j CW + c.  A stage's butterflies are numbered column-fastest,
+// so the lanes of a half-wave touch 32 consecutive columns of one row (no
+// bank conflicts, one shared twiddle), and every index is a shift or mask of
+// the butterfly number.
+constexpr int kHotMaxPts = 8192;  // points per K1/K3 workgroup (16 per thread)
+constexpr int hot_cw(int p1) {
+  int c = 1;
+  while (2 * c * p1 <= kMaxWG && 2 * c <= kHotP2) c *= 2;
+  return c < 32 ? 32 : c;
+}
 constexpr int ilog2c(int v) { return v <= 1 ? 0 : 1 + ilog2c(v >> 1); }
-// Column tile of the general kernels: the largest power of two with
-// cw P1 <= 4096.
+// Column tile of the general kernels (the spectrum pass runs on the plan's
+// geometry): the largest power of two with cw P1 <= 4096.
 constexpr int generic_cw(int p1) {
   int c = 1;
   while (2 * c * p1 <= kMaxWG && 2 * c <= kHotP2) c *= 2;
   return c;
 }
+
+// One radix-R stage of N-point column FFTs over the CW columns of a
+// column-major tile; the tail of the last butterfly round is masked when
+// CW N / R is not a multiple of the workgroup size.
+template <bool INV, int R, int N, int NS, int CW>
+__device__ __forceinline__ void ct_stage_cm(cx<float>* buf, const cx<float>* tw) {
+  constexpr int Q = N / R, TOT = CW * Q, NB = (TOT + kThreads - 1) / kThreads, LCW = ilog2c(CW);
+  constexpr bool FULL = NB * kThreads == TOT;
+  cx<float> v[NB][R];
+#pragma unroll
+  for (int u = 0; u < NB; u++) {
+    const int bf = threadIdx.x + u * kThreads;
+    if (FULL || bf < TOT) {
+      const int c = bf & (CW - 1), j = bf >> LCW, k = j % NS;
+#pragma unroll
+      for (int r = 0; r < R; r++) v[u][r] = buf[(j + r * Q) * CW + c];
+      if (NS > 1) {
+#pragma unroll
+        for (int r = 1; r < R; r++) {
+          cx<float> w = tw[(r - 1) * NS + k];
+          if (INV) w = cconj(w);
+          v[u][r] = cmul(v[u][r], w);
+        }
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < NB; u++) {
+    const int bf = threadIdx.x + u * kThreads;
+    if (FULL || bf < TOT) {
+      const int c = bf & (CW - 1), j = bf >> LCW, k = j % NS;
+      dft_r<float, INV, R>(v[u]);
+      const int idx = (j / NS) * NS * R + k;
+#pragma unroll
+      for (int r = 0; r < R; r++) buf[(idx + r * NS) * CW + c] = v[u][r];
+    }
+  }
+  __syncthreads();
+}
+
+template <bool INV, int N, int CW, int NS = 1, int OFF = 0>
+__device__ __forceinline__ void ct_fft_cm(cx<float>* buf, const cx<float>* st) {
+  if constexpr (NS < N) {
+    constexpr int R = next_radix(N / NS);
+    ct_stage_cm<INV, R, N, NS, CW>(buf, st + OFF);
+    ct_fft_cm<INV, N, CW, NS * R, OFF + (R - 1) * NS>(buf, st);
+  }
+}
+
+// Blocks are taken in an XCD-aware order: the hardware deals consecutive
+// block ids round-robin over the 8 XCDs, and the remap gives each XCD a
+// contiguous range of (row, column block) tiles, so the pieces of one row
+// run together on one XCD.  A row's input is then read from HBM once and
+// its mirrored images (each sample appears up to three times in the even
+// extension) come from that XCD's L2: K1's fetch drops from 28.4 to 7.8 GB
+// per apply on the 64-TOD benchmark.
+template <int P1>
+__global__ void __launch_bounds__(kThreads, 2) k1_hot_kernel(const Seg* __restrict__ segs, int nseg,
+                                                              const float* __restrict__ in,
+                                                              cx<float>* __restrict__ tbuf,
+                                                              const cx<float>* __restrict__ stab_g,
+                                                              int64_t nblk) {
+  constexpr int CW = hot_cw(P1), LCW = ilog2c(CW), NPTS = CW * P1;
+  constexpr int P = P1 * kHotP2;
+  static_assert(NPTS <= kHotMaxPts && kHotP2 % CW == 0, "K1 tile");
+  extern __shared__ unsigned char smem_raw[];
+  const int64_t per = ((int64_t)gridDim.x + 7) / 8;
+  const int64_t bid = (int64_t)(blockIdx.x % 8) * per + blockIdx.x / 8;
+  if (bid >= nblk) return;
+  const int s = find_seg(segs, nseg, bid, 1);
+  const Seg sg = segs[s];
+  const int local = (int)(bid - sg.base1);
+  const int row = local / sg.per1, jb = local - row * sg.per1;
+  const int m = sg.n - 1;
+  cx<float>* buf = reinterpret_cast<cx<float>*>(smem_raw);  // [P1][CW]
+  cx<float>* st = buf + NPTS;                                // [P1] stage table
+  cx<float>* F = st + P1;                                    // [1024] w_2P^l
+  cx<float>* Ct = F + (1 << kFineBits);                      // [4 P1] w_2P^(1024 h)
+  const cx<float>* twF = reinterpret_cast<const cx<float>*>(sg.tw_ptr);
+  for (int e = threadIdx.x; e < P1 - 1; e += kThreads) st[e] = stab_g[e];
+  for (int e = threadIdx.x; e < (1 << kFineBits); e += kThreads) F[e] = twF[e];
+  for (int e = threadIdx.x; e < 4 * P1; e += kThreads) Ct[e] = twF[(1 << kFineBits) + e];
+  const float* x = in + sg.in_off + (int64_t)row * sg.in_stride;
+  const int j2_0 = jb * CW;
+  // real input a_i, i = 2 (P2 j1 + j2) + w, from the even extension on
+  // [-m, 2m]; reals 2 (j1 CW + c) + {0, 1} of the tile are consecutive.
+  // A thread's w is the same for every u and j1 grows by kThreads / 2CW, so
+  // i is affine in u.  The extension's sample is x[m - |m - |i - m||], and
+  // past 3m that index is negative: as a 32-bit buffer offset it lies past
+  // the row's bytes, and the buffer load returns the padding's zero.
+  // (Wide tiles of short columns, 2CW > kThreads, compute i per u.)
+  constexpr int NR = 2 * NPTS, NV = (NR + kThreads - 1) / kThreads;
+  const __amdgpu_buffer_rsrc_t xrs =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x), (short)0, (int)((m + 1) * 4), 0x00020000);
+  float val[NV];
+  if constexpr (kThreads % (2 * CW) == 0) {
+    constexpr int DI = 2 * kHotP2 * (kThreads / (2 * CW));  // i step per u
+    const int t0 = 2 * (kHotP2 * ((int)threadIdx.x >> (LCW + 1)) + j2_0) + ((int)threadIdx.x & (2 * CW - 1)) - m;
+#pragma unroll
+    for (int u = 0; u < NV; u++) {
+      const int t = t0 + u * DI;
+      const int xi = m - abs(m - abs(t));
+      const float v = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, (uint32_t)xi * 4u, 0u, 0));
+      val[u] = (NV * kThreads == NR || (int)threadIdx.x + u * kThreads < NR) ? v : 0.f;
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < NV; u++) {
+      const int idx = threadIdx.x + u * kThreads;
+      const int t = 2 * (kHotP2 * (idx >> (LCW + 1)) + j2_0) + (idx & (2 * CW - 1)) - m;
+      const int xi = m - abs(m - abs(t));
+      const float v = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, (uint32_t)xi * 4u, 0u, 0));
+      val[u] = (NV * kThreads == NR || idx < NR) ? v : 0.f;
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < NV; u++) {
+    const int idx = threadIdx.x + u * kThreads;
+    if (NV * kThreads == NR || idx < NR) reinterpret_cast<float*>(buf)[idx] = val[u];
+  }
+  __syncthreads();
+  ct_fft_cm<false, P1, CW>(buf, st);
+  cx<float>* trow = tbuf + sg.t_off + (int64_t)row * sg.t_stride;
+  constexpr int NO = (NPTS + kThreads - 1) / kThreads;
+  // The thread's column c is the same for every u (kThreads is a multiple of
+  // CW) and k1 grows by kThreads / CW per step, so the twiddles w^(2 (j2_0+c) k1)
+  // form a geometric sequence: one complex multiply per step, re-seeded from
+  // the exact tables every 4 steps so FP32 rounding does not build up.
+  if constexpr (kThreads % CW == 0) {
+    const int c = threadIdx.x & (CW - 1), j2 = j2_0 + c;
+    const cx<float> step = tw2P(F, Ct, 2 * ((j2 * (kThreads / CW)) % P));
+    cx<float> tw{1.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < NO; u++) {
+      const int idx = threadIdx.x + u * kThreads;
+      if (NO * kThreads != NPTS && idx >= NPTS) break;
+      const int k1 = idx >> LCW;
+      if ((u & 3) == 0) tw = tw2P(F, Ct, 2 * ((j2 * k1) % P));  // < 2^11 * 2^8
+      trow[k1 * kHotP2 + j2] = cmul(buf[idx], tw);
+      tw = cmul(tw, step);
+    }
+  } else {  // CW > kThreads (short columns): the column changes with u
+#pragma unroll
+    for (int u = 0; u < NO; u++) {
+      const int idx = threadIdx.x + u * kThreads;
+      if (NO * kThreads != NPTS && idx >= NPTS) break;
+      const int k1 = idx >> LCW, c = idx & (CW - 1);
+      const int a = ((j2_0 + c) * k1) % P;  // < 2^11 * 2^8
+      trow[k1 * kHotP2 + j2_0 + c] = cmul(buf[idx], tw2P(F, Ct, 2 * a));
+    }
+  }
+}
+
+template <int P1>
+__global__ void __launch_bounds__(kThreads, 2) k3_hot_kernel(const Seg* __restrict__ segs, int nseg,
+                                                              const cx<float>* __restrict__ tbuf,
+                                                              float* __restrict__ out,
+                                                              const cx<float>* __restrict__ stab_g) {
+  constexpr int CW = hot_cw(P1), LCW = ilog2c(CW), NPTS = CW * P1;
+  constexpr int P = P1 * kHotP2;
+  static_assert(NPTS <= kHotMaxPts && kHotP2 % CW == 0, "K3 tile");
+  extern __shared__ unsigned char smem_raw[];
+  const int s = find_seg(segs, nseg, blockIdx.x, 3);
+  const Seg sg = segs[s];
+  const int local = (int)((int64_t)blockIdx.x - sg.base3);
+  const int row = local / sg.per1, jb = local - row * sg.per1;
+  const int m = sg.n - 1;
+  cx<float>* buf = reinterpret_cast<cx<float>*>(smem_raw);  // [P1][CW]
+  cx<float>* st = buf + NPTS;                                // [P1] stage table
+  for (int e = threadIdx.x; e < P1 - 1; e += kThreads) st[e] = stab_g[e];
+  const cx<float>* trow = tbuf + sg.t_off + (int64_t)row * sg.t_stride;
+  const int j2_0 = jb * CW;
+  {
+    constexpr int NV = (NPTS + kThreads - 1) / kThreads;
+    cx<float> v[NV];
+#pragma unroll
+    for (int u = 0; u < NV; u++) {
+      const int idx = threadIdx.x + u * kThreads;
+      if (NV * kThreads == NPTS || idx < NPTS) v[u] = trow[(idx >> LCW) * kHotP2 + j2_0 + (idx & (CW - 1))];
+    }
+#pragma unroll
+    for (int u = 0; u < NV; u++) {
+      const int idx = threadIdx.x + u * kThreads;
+      if (NV * kThreads == NPTS || idx < NPTS) buf[idx] = v[u];
+    }
+  }
+  __syncthreads();
+  ct_fft_cm<true, P1, CW>(buf, st);
+  const float scale = 1.f / (float)P;
+  const bool halve = sg.flags & 1;
+  float* y = out + sg.out_off + (int64_t)row * sg.out_stride;
+  constexpr int NR = 2 * NPTS, NO = (NR + kThreads - 1) / kThreads;
+#pragma unroll
+  for (int u = 0; u < NO; u++) {
+    const int idx = threadIdx.x + u * kThreads;
+    if (NO * kThreads != NR && idx >= NR) break;
+    const int j1 = idx >> (LCW + 1), w = idx & (2 * CW - 1);
+    const int k = 2 * (kHotP2 * j1 + j2_0) + w - m;
+    if (k >= 0 && k <= m) {
+      float v = reinterpret_cast<const float*>(buf)[idx] * scale;
+      if (halve && (k == 0 || k == m)) v *= 0.5f;
+      y[k] = v;
+    }
+  }
+}
+
+// Column lengths of the hot path: every 5-smooth P1 in [2, 256].
 constexpr int kHotP1[] = {2,   3,   4,   5,   6,   8,   9,   10,  12,  15,  16,  18,  20,  24,  25,  27,  30,
                           32,  36,  40,  45,  48,  50,  54,  60,  64,  72,  75,  80,  81,  90,  96,  100, 108,
                           120, 125, 128, 135, 144, 150, 160, 162, 180, 192, 200, 216, 225, 240, 243, 250, 256};
@@ -435,6 +1060,57 @@ int hot_p1_index(int p1) {
   for (int i = 0; i < kNumHotP1; i++)
     if (kHotP1[i] == p1) return i;
   return -1;
+}
+
+// LDS of the hot K1 (tile, stage table, fine/coarse tables) and K3 (tile,
+// stage table).
+size_t hot13_lds(int p1, int which) {
+  return (size_t)(hot_cw(p1) * p1 + p1 + (which == 1 ? (1 << kFineBits) + 4 * p1 : 0)) * sizeof(cx<float>);
+}
+
+// Stage table of an N-point mixed-radix FFT (fill_stage_table_mx order),
+// computed in FP64.
+__global__ void mixed_stage_table_kernel(cx<float>* out, int N) {
+  int Ns = 1, off = 0;
+  while (Ns < N) {
+    const int R = next_radix(N / Ns), cnt = (R - 1) * Ns;
+    for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < cnt; e += gridDim.x * blockDim.x) {
+      const int r = e / Ns + 1, k = e - (r - 1) * Ns;
+      double sn, cs;
+      sincospi(-2.0 * (double)(k * r) / (double)(R * Ns), &sn, &cs);
+      out[off + e] = {(float)cs, (float)sn};
+    }
+    off += cnt;
+    Ns *= R;
+  }
+}
+
+// Twiddle tables of the hot K2 path, computed in FP64: the stage table of a
+// 2^11-point FFT (fill_stage_table order) and, per P, w_2P^l (l < 1024) then
+// w_2P^(1024 h) (h < 2P / 1024).
+__global__ void hot_tables_kernel(cx<float>* out, int64_t P, int stage_l2) {
+  if (stage_l2 > 0) {  // stage table of a 2^stage_l2-point FFT
+    int Ns = 1, rem = stage_l2, off = 0;
+    while (rem > 0) {
+      const int lr = stage_lr(rem), R = 1 << lr, cnt = (R - 1) * Ns, mul = 1 << (rem - lr);
+      for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < cnt; e += gridDim.x * blockDim.x) {
+        int r = e / Ns + 1, k = e - (r - 1) * Ns;
+        double sn, cs;
+        sincospi(-2.0 * (double)((int64_t)k * r * mul) / (double)(1 << stage_l2), &sn, &cs);
+        out[off + e] = {(float)cs, (float)sn};
+      }
+      off += cnt;
+      Ns <<= lr; rem -= lr;
+    }
+    return;
+  }
+  const int64_t nF = 1 << kFineBits, nC = 2 * P / nF;
+  for (int64_t e = blockIdx.x * blockDim.x + threadIdx.x; e < nF + nC; e += gridDim.x * blockDim.x) {
+    int64_t t = e < nF ? e : (e - nF) * nF;  // exponent of w_2P
+    double sn, cs;
+    sincospi(-(double)t / (double)P, &sn, &cs);
+    out[e] = {(float)cs, (float)sn};
+  }
 }
 
 // ---- K3: inverse column FFTs + output -------------------------------------
@@ -546,7 +1222,7 @@ Geometry hot_geometry(int p1) {
 }
 
 Geometry geometry(int64_t P_min, int elem_bytes, bool mixed = false) {
-  if (mixed && P_min > kHotP2) {  // a length class of the 2^11-point-row engine
+  if (mixed && P_min > kHotP2) {
     const int64_t need = (P_min + kHotP2 - 1) / kHotP2;
     for (int i = 0; i < kNumHotP1; i++)
       if (kHotP1[i] >= need) return hot_geometry(kHotP1[i]);
@@ -576,6 +1252,15 @@ void allow_big_lds(K kernel) {
                             kMaxLds);
 }
 
+template <int I = 0>
+void allow_lds_hot13() {
+  if constexpr (I < kNumHotP1) {
+    allow_big_lds(k1_hot_kernel<kHotP1[I]>);
+    allow_big_lds(k3_hot_kernel<kHotP1[I]>);
+    allow_lds_hot13<I + 1>();
+  }
+}
+
 void allow_lds_all() {
   static bool done = false;
   if (done) return;
@@ -601,7 +1286,8 @@ void allow_lds_all() {
   allow_big_lds(k3_kernel<double, double, kFilter>);
   allow_big_lds(k3_kernel<float, float, kBlue>);
   allow_big_lds(k3_kernel<double, double, kBlue>);
-  allow_rows_lds();
+  allow_big_lds(k2_hot_kernel);
+  allow_lds_hot13();
   (void)hipGetLastError();  // an unsupported attribute must not poison later launch checks
 }
 
@@ -635,29 +1321,28 @@ struct mk_filt_plan {
   int nseg = 0;
   int elem_bytes = 4;  // 4: FP32 spectra and T buffer, 8: FP64
   std::vector<Seg> h_segs;
+  Seg* d_segs = nullptr;
   int64_t n1 = 0, n2 = 0;  // total K1/K3 items, K2 items
-  int64_t t_elems = 0, s_elems = 0;  // complex values of the work buffer, reals of the spectra
+  int64_t t_elems = 0, s_elems = 0;
   void* tbuf = nullptr;    // complex
   bool tbuf_owned = true;  // false: the caller's buffer (mk_filt_plan_set_work)
-  void* spec = nullptr;    // real: 2 (P+2) per row on the 2^11-row path, P+1 on the general one
-  size_t lds1 = 0, lds2 = 0;  // LDS of the general kernels
+  void* spec = nullptr;    // real, P+1 per row
+  size_t lds1 = 0, lds2 = 0;
   bool have_spec = false;
   std::vector<char> borrowed;
-  // Segments on the 2^11-row path (one list for the row pass and one grouped
-  // by column count for the column passes, a launch per count) and the rest,
-  // each list with its own work-item numbering.
+  // FP32 K2 split: segments on the hot path (rows of 2^11, P1 <= 256) and the
+  // rest, each list with its own K2 numbering; twiddle tables for the hot path
   Seg* d_hot = nullptr;
-  Seg* d_hotc = nullptr;
   Seg* d_cold = nullptr;
+  Seg* d_hot13 = nullptr;   // hot segments grouped by column length, K1/K3 numbering per group
   int nhot = 0, ncold = 0;
   int64_t n2hot = 0, n2cold = 0, n1cold = 0;
-  int g_off[kNumQ1] = {0}, g_cnt[kNumQ1] = {0};  // per column count (kQ1 index)
-  int64_t g_n1[kNumQ1] = {0};
-  // twiddle tables in the plan's precision, and in FP64 for the spectrum pass
-  // of an FP32 plan (freed after it): the common ones, then one per count
-  void* tw = nullptr;
-  int64_t g_tab[kNumQ1] = {0};  // element offset of a count's table
-  int64_t tw_elems = 0, tw_all = 0;  // complex elements without / with the end-mode phases
+  int g_off[kNumHotP1] = {0}, g_cnt[kNumHotP1] = {0};  // per column length (kHotP1 index)
+  int64_t g_n1[kNumHotP1] = {0};
+  int64_t g_stab[kNumHotP1] = {0};  // offset of that length's stage table in tw_tab
+  // stage tables of 2^1..2^11 points (2^l - 2 offsets), then per-P fine/coarse
+  // tables, then the mixed-radix stage tables of the hot column lengths
+  void* tw_tab = nullptr;
 };
 
 namespace {
@@ -675,20 +1360,31 @@ int ensure_tbuf(const mk_filt_plan* cp) {
   return MK_OK;
 }
 
-// Uploads the segment lists; eb: precision of the passes they number (the
-// column tile depends on it).
-int upload_lists(mk_filt_plan* p, int eb) {
-  std::vector<Seg> hot, cold, hotc;
+bool hot_shape(const Seg& s) { return s.l2 == kHotL2 && hot_p1_index(s.p1) >= 0; }
+bool is_hot(const mk_filt_plan* p, const Seg& s) {
+  return p->elem_bytes == 4 && hot_shape(s) && s.tw_ptr != nullptr;
+}
+
+int upload(mk_filt_plan* p) {
+  if (p->nseg && hipMemcpy(p->d_segs, p->h_segs.data(), p->nseg * sizeof(Seg), hipMemcpyHostToDevice) != hipSuccess) {
+    mk::set_error("filter plan: descriptor upload failed");
+    return MK_ERR_HIP;
+  }
+  if (p->elem_bytes != 4) return MK_OK;
+  std::vector<Seg> hot, cold, hot13;
   int64_t b_hot = 0, b_cold2 = 0, b_cold1 = 0;
   for (const Seg& s0 : p->h_segs) {
     Seg s = s0;
-    if (s.hot) {
-      s.tw_off = p->g_tab[q1_index(s.q1)];
-      s.per2 = (s.q1 + 1) / 2;  // pairs (k1, q1-k1), k1 = 1..; column 0 (+ q1/2) in item 0
+    if (is_hot(p, s)) {
+      s.per2 = (s.p1 + 1) / 2;  // pairs (k1, P1-k1), k1 = 1..; column 0 (+ P1/2) in item 0
       s.base2 = b_hot;
       b_hot += (int64_t)s.rows * s.per2;
       hot.push_back(s);
     } else {
+      if (s.l1 < 0) {
+        mk::set_error("filter plan: column length %d is only supported on the FP32 hot path", s.p1);
+        return MK_ERR_ARG;
+      }
       s.base2 = b_cold2;
       b_cold2 += (int64_t)s.rows * s.per2;
       s.base1 = s.base3 = b_cold1;
@@ -696,17 +1392,18 @@ int upload_lists(mk_filt_plan* p, int eb) {
       cold.push_back(s);
     }
   }
-  for (int l = 0; l < kNumQ1; l++) {
-    p->g_off[l] = (int)hotc.size();
+  for (int l = 0; l < kNumHotP1; l++) {
+    p->g_off[l] = (int)hot13.size();
     int64_t b = 0;
     for (const Seg& s0 : hot)
-      if (s0.q1 == kQ1[l]) {
+      if (s0.p1 == kHotP1[l]) {
         Seg s = s0;
+        s.per1 = kHotP2 / hot_cw(s.p1);  // the hot K1/K3 tile is wider than the general one
         s.base1 = s.base3 = b;
-        b += (int64_t)s.rows * (eb == 4 ? col_blocks<float>(s.q1) : col_blocks<double>(s.q1));
-        hotc.push_back(s);
+        b += (int64_t)s.rows * s.per1;
+        hot13.push_back(s);
       }
-    p->g_cnt[l] = (int)hotc.size() - p->g_off[l];
+    p->g_cnt[l] = (int)hot13.size() - p->g_off[l];
     p->g_n1[l] = b;
   }
   p->nhot = (int)hot.size();
@@ -715,86 +1412,81 @@ int upload_lists(mk_filt_plan* p, int eb) {
   p->n2cold = b_cold2;
   p->n1cold = b_cold1;
   if ((p->nhot && hipMemcpy(p->d_hot, hot.data(), hot.size() * sizeof(Seg), hipMemcpyHostToDevice) != hipSuccess) ||
-      (p->nhot && hipMemcpy(p->d_hotc, hotc.data(), hotc.size() * sizeof(Seg), hipMemcpyHostToDevice) != hipSuccess) ||
-      (p->ncold && hipMemcpy(p->d_cold, cold.data(), cold.size() * sizeof(Seg), hipMemcpyHostToDevice) != hipSuccess)) {
+      (p->nhot &&
+       hipMemcpy(p->d_hot13, hot13.data(), hot13.size() * sizeof(Seg), hipMemcpyHostToDevice) != hipSuccess) ||
+      (p->ncold &&
+       hipMemcpy(p->d_cold, cold.data(), cold.size() * sizeof(Seg), hipMemcpyHostToDevice) != hipSuccess)) {
     mk::set_error("filter plan: descriptor upload failed");
     return MK_ERR_HIP;
   }
   return MK_OK;
 }
-int upload(mk_filt_plan* p) { return upload_lists(p, p->elem_bytes); }
 
-// The tables a plan uses: the common ones, then one per column count, then
-// the end-mode phases per row length (of one column count).
-void layout_tables(mk_filt_plan* p) {
-  p->tw_elems = 0;
-  for (Seg& s : p->h_segs) {
-    if (!s.hot) continue;
-    if (p->tw_elems == 0) p->tw_elems = kTwCommon;
-    const int i = q1_index(s.q1);
-    if (!p->g_tab[i]) {
-      p->g_tab[i] = p->tw_elems;
-      p->tw_elems += q1_table_elems(s.q1);
-    }
-  }
-  p->tw_all = p->tw_elems;
-  for (size_t i = 0; i < p->h_segs.size(); i++) {
-    Seg& s = p->h_segs[i];
-    if (!s.hot) continue;
-    s.em_off = 0;
-    for (size_t k = 0; k < i && !s.em_off; k++) {
-      const Seg& o = p->h_segs[k];
-      if (o.hot && o.n == s.n && o.q1 == s.q1) s.em_off = o.em_off;
-    }
-    if (!s.em_off) {
-      s.em_off = p->tw_all;
-      p->tw_all += end_phase_elems(s.q1);
-    }
-  }
-}
+const cx<float>* stage_tab(const mk_filt_plan* p, int l) { return (const cx<float>*)p->tw_tab + ((1 << l) - 2); }
 
-// Builds the twiddle tables in precision T into tab (tw_elems values).
-template <typename T>
-int build_tables(const mk_filt_plan* p, void* tab, hipStream_t st) {
-  bool first = true;
-  for (int i = 0; i < kNumQ1; i++)
-    if (p->g_tab[i]) {
-      launch_col_tables<T>(kQ1[i], first ? (cx<T>*)tab : nullptr, (cx<T>*)tab + p->g_tab[i], st);
-      first = false;
-    }
-  return mk::check_launch("col_tables_kernel");
-}
-template <typename T>
-int build_end_phases(const mk_filt_plan* p, hipStream_t st) {
-  int64_t next = p->tw_elems;
+// Builds the hot-path twiddle tables of an FP32 plan and points each hot
+// segment at its P's tables.
+int build_hot_tables(mk_filt_plan* p) {
+  std::vector<int64_t> Ps;
+  std::vector<int> p1s;
   for (const Seg& s : p->h_segs)
-    if (s.hot && s.em_off == next) {  // a length's first segment
-      launch_end_phases<T>((cx<T>*)p->tw + next, s.n, s.q1, st);
-      next += end_phase_elems(s.q1);
+    if (hot_shape(s)) {
+      const int64_t P = (int64_t)s.p1 * kHotP2;
+      if (std::find(Ps.begin(), Ps.end(), P) == Ps.end()) Ps.push_back(P);
+      if (std::find(p1s.begin(), p1s.end(), s.p1) == p1s.end()) p1s.push_back(s.p1);
     }
-  return mk::check_launch("end_phase_kernel");
+  if (Ps.empty()) return MK_OK;
+  std::vector<int64_t> offs;
+  int64_t tot = 2 * kHotP2;  // stage tables of 2^1 .. 2^11 points first
+  for (int64_t P : Ps) {
+    offs.push_back(tot);
+    tot += (1 << kFineBits) + 2 * P / (1 << kFineBits);
+  }
+  for (int v : p1s) {
+    p->g_stab[hot_p1_index(v)] = tot;
+    tot += v;  // v - 1 entries, rounded up
+  }
+  if (hipMalloc(&p->tw_tab, tot * sizeof(cx<float>)) != hipSuccess) {
+    p->tw_tab = nullptr;
+    mk::set_error("filter plan: twiddle table allocation failed");
+    return MK_ERR_ALLOC;
+  }
+  cx<float>* base = (cx<float>*)p->tw_tab;
+  for (int l = 1; l <= kHotL2; l++) hot_tables_kernel<<<8, 256>>>(base + ((1 << l) - 2), 0, l);
+  for (size_t i = 0; i < Ps.size(); i++) hot_tables_kernel<<<64, 256>>>(base + offs[i], Ps[i], 0);
+  for (int v : p1s) mixed_stage_table_kernel<<<1, 256>>>(base + p->g_stab[hot_p1_index(v)], v);
+  int r = mk::check_launch("hot_tables_kernel");
+  if (r) return r;
+  MK_HIP(hipDeviceSynchronize());
+  for (Seg& s : p->h_segs)
+    if (hot_shape(s)) {
+      const int64_t P = (int64_t)s.p1 * kHotP2;
+      size_t i = std::find(Ps.begin(), Ps.end(), P) - Ps.begin();
+      s.tw_ptr = base + offs[i];
+    }
+  return MK_OK;
 }
 
 void free_filt(mk_filt_plan* p) {
   if (!p) return;
+  if (p->d_segs) (void)hipFree(p->d_segs);
   if (p->d_hot) (void)hipFree(p->d_hot);
-  if (p->d_hotc) (void)hipFree(p->d_hotc);
+  if (p->d_hot13) (void)hipFree(p->d_hot13);
   if (p->d_cold) (void)hipFree(p->d_cold);
-  if (p->tw) (void)hipFree(p->tw);
+  if (p->tw_tab) (void)hipFree(p->tw_tab);
   if (p->tbuf && p->tbuf_owned) (void)hipFree(p->tbuf);
   if (p->spec) (void)hipFree(p->spec);
   delete p;
 }
 
 // desc per segment: {rows, n, in_off, in_stride, out_off, out_stride}
-// mixed: FP32 filter plans, whose geometry is reported in length classes.
-// hot: rows longer than 2^11 * 2/3 samples and up to 2^19 take the
-// 2^11-point-row engine.
+// mixed: FP32 filter plans whose rows may take the hot path's 5-smooth
+// column lengths.
 // p1 (may be null): per segment a hot column length chosen by the caller
 // (0 = the default, the smallest one that fits).
 int build_segs(int nseg, const int64_t* desc, int eb, bool filter, std::vector<Seg>& segs, int64_t* n1,
                int64_t* n2, int64_t* t_elems, int64_t* s_elems, size_t* lds1, size_t* lds2, bool mixed = false,
-               const int32_t* p1 = nullptr, bool hot = false) {
+               const int32_t* p1 = nullptr) {
   segs.clear();
   int64_t b1 = 0, b2 = 0, toff = 0, soff = 0;
   size_t l1max = 0, l2max = 0;
@@ -807,7 +1499,6 @@ int build_segs(int nseg, const int64_t* desc, int eb, bool filter, std::vector<S
     int64_t m = n - 1;
     const int64_t P_min = filter ? (3 * m + 2) / 2 : 2 * m + 1;
     Geometry g = geometry(P_min, eb, mixed);
-    const int p1_min = g.p1;
     if (p1 && p1[i] > 0) {
       MK_REQUIRE(mixed && hot_p1_index(p1[i]) >= 0, MK_ERR_ARG,
                  "segment %d: column length %d is not one of the FP32 hot lengths", i, (int)p1[i]);
@@ -819,78 +1510,88 @@ int build_segs(int nseg, const int64_t* desc, int eb, bool filter, std::vector<S
     Seg s{};
     s.in_off = d[2]; s.in_stride = d[3]; s.out_off = d[4]; s.out_stride = d[5];
     s.rows = (int32_t)rows; s.n = (int32_t)n; s.l1 = g.l1; s.l2 = g.l2; s.cw = g.cw; s.flags = 0; s.p1 = g.p1;
-    // the engine's own length: 2^11 q1 >= n, and for a longer class than the
-    // default two thirds of its columns
-    s.q1 = 0;
-    if (hot && filter && P_min > kHotP2) {
-      const int64_t cls = p1 && p1[i] > p1_min ? mk::cdiv(2 * (int64_t)p1[i], 3) * kHotP2 : 0;
-      s.q1 = q1_at_least(std::max(m + 1, cls));
-    }
-    s.hot = s.q1 > 0;
-    const int64_t P = s.hot ? (int64_t)s.q1 * kHotP2 : g.P;
-    const int64_t s_row = s.hot ? 2 * (P + 2) : P + 1;
-    s.t_off = toff; s.t_stride = P;
-    s.s_off = soff; s.s_stride = filter ? s_row : 0;
+    s.t_off = toff; s.t_stride = g.P;
+    s.s_off = soff; s.s_stride = filter ? g.P + 1 : 0;
     s.per1 = (int32_t)((int64_t(1) << g.l2) / g.cw);
     s.r2 = k2_r2(g, 8, filter);  // same grouping for FP32 and FP64 passes
     s.per2 = (int32_t)mk::cdiv(filter ? g.p1 / 2 + 1 : g.p1, s.r2);
     s.base1 = b1; s.base2 = b2; s.base3 = b1;
     b1 += rows * s.per1;
     b2 += rows * s.per2;
-    toff += rows * P;
-    soff += filter ? rows * s_row : P;
-    if (!s.hot) {
-      l1max = std::max(l1max, lds_k13(g, eb));
-      l2max = std::max(l2max, lds_k2(g, eb, filter));
-    }
+    toff += rows * g.P;
+    soff += filter ? rows * (g.P + 1) : g.P;
+    l1max = std::max(l1max, lds_k13(g, eb));
+    l2max = std::max(l2max, lds_k2(g, eb, filter));
     MK_REQUIRE(l1max <= (size_t)kMaxLds && l2max <= (size_t)kMaxLds, MK_ERR_ARG,
                "segment %d: n=%lld needs more LDS than the %d-byte budget at %d-byte precision", i,
                (long long)n, kMaxLds, eb);
     segs.push_back(s);
   }
-  for (Seg& s : segs) {  // behind the rows: one value per row of the 2^11-row path
-    s.e_off = toff;
-    if (s.hot) toff += s.rows;
-  }
   *n1 = b1; *n2 = b2; *t_elems = toff; *s_elems = soff; *lds1 = l1max; *lds2 = l2max;
   return MK_OK;
 }
 
-// Spectrum pass of the general path in arithmetic type T into spectra of type
-// TS; lds1/lds2 sized for T.
+// Spectrum pass in arithmetic type T into spectra of type TS; tb holds
+// rows*P complex<T>; lds1/lds2 sized for T.
 template <typename T, typename TS>
 void launch_fspec(mk_filt_plan* p, const void* wdct, void* tb, size_t lds1, size_t lds2, hipStream_t st) {
-  k1_kernel<T, double, kFSpec><<<(unsigned)p->n1cold, kThreads, lds1, st>>>(p->d_cold, p->ncold, (const double*)wdct,
-                                                                            (cx<T>*)tb);
-  k2_kernel<T, TS, kFSpec><<<(unsigned)p->n2cold, kThreads, lds2, st>>>(p->d_cold, p->ncold, (cx<T>*)tb);
+  k1_kernel<T, double, kFSpec><<<(unsigned)p->n1, kThreads, lds1, st>>>(p->d_segs, p->nseg, (const double*)wdct,
+                                                                        (cx<T>*)tb);
+  k2_kernel<T, TS, kFSpec><<<(unsigned)p->n2, kThreads, lds2, st>>>(p->d_segs, p->nseg, (cx<T>*)tb);
 }
 
-// The 2^11-row path's column passes over every column count of the plan.
-template <typename T>
-void launch_hot_fwd(const mk_filt_plan* p, int mode, const void* in, cx<T>* tb, const cx<T>* tw, int comp,
-                    hipStream_t st) {
-  for (int i = 0; i < kNumQ1; i++)
-    if (p->g_n1[i])
-      launch_cols_fwd<T>(kQ1[i], mode, p->d_hotc + p->g_off[i], p->g_cnt[i], p->g_n1[i], in, tb,
-                         tw, tw + p->g_tab[i] + kQ1[i] * kRowTw, nullptr, comp, st);
+template <int I>
+void launch_hot13(const mk_filt_plan* p, int which, const float* in, float* out, hipStream_t st) {
+  constexpr int P1 = kHotP1[I];
+  const Seg* segs = p->d_hot13 + p->g_off[I];
+  const unsigned grid = (unsigned)p->g_n1[I];
+  const cx<float>* stab = (const cx<float>*)p->tw_tab + p->g_stab[I];
+  if (which == 1)  // XCD-aware block order: the grid is rounded up to a multiple of 8 XCDs
+    k1_hot_kernel<P1><<<(unsigned)(mk::cdiv(grid, 8) * 8), kThreads, hot13_lds(P1, 1), st>>>(
+        segs, p->g_cnt[I], in, (cx<float>*)p->tbuf, stab, (int64_t)grid);
+  else
+    k3_hot_kernel<P1><<<grid, kThreads, hot13_lds(P1, 3), st>>>(segs, p->g_cnt[I], (const cx<float>*)p->tbuf, out,
+                                                             stab);
+}
+
+template <int I = 0>
+void launch_hot13_idx(const mk_filt_plan* p, int idx, int which, const float* in, float* out, hipStream_t st) {
+  if constexpr (I < kNumHotP1) {
+    if (idx == I) launch_hot13<I>(p, which, in, out, st);
+    else launch_hot13_idx<I + 1>(p, idx, which, in, out, st);
+  }
+}
+
+void launch_hot13_all(const mk_filt_plan* p, int which, const float* in, float* out, hipStream_t st) {
+  for (int i = 0; i < kNumHotP1; i++)
+    if (p->g_cnt[i] && p->g_n1[i]) launch_hot13_idx(p, i, which, in, out, st);
 }
 
 template <typename T, typename TIO>
 void launch_filter(const mk_filt_plan* p, const TIO* in, TIO* out, hipStream_t st) {
-  cx<T>* tb = (cx<T>*)p->tbuf;
-  const cx<T>* tw = (const cx<T>*)p->tw;
-  launch_hot_fwd<T>(p, kFilter, in, tb, tw, 0, st);
-  if (p->n1cold)
-    k1_kernel<T, TIO, kFilter><<<(unsigned)p->n1cold, kThreads, p->lds1, st>>>(p->d_cold, p->ncold, in, tb);
-  if (p->n2hot) launch_rows<T>(kFilter, p->d_hot, p->nhot, p->n2hot, tb, tw, 0, false, st);
-  if (p->n2cold)
-    k2_kernel<T, T, kFilter><<<(unsigned)p->n2cold, kThreads, p->lds2, st>>>(p->d_cold, p->ncold, tb);
-  for (int i = 0; i < kNumQ1; i++)
-    if (p->g_n1[i])
-      launch_cols_inv<T>(kQ1[i], kFilter, p->d_hotc + p->g_off[i], p->g_cnt[i], p->g_n1[i], tb, out,
-                         tw, tw + p->g_tab[i] + kQ1[i] * kRowTw, nullptr, st);
-  if (p->n1cold)
-    k3_kernel<T, TIO, kFilter><<<(unsigned)p->n1cold, kThreads, p->lds1, st>>>(p->d_cold, p->ncold, tb, out);
+  if constexpr (sizeof(T) == 4) {
+    if (p->nhot + p->ncold == p->nseg) {
+      launch_hot13_all(p, 1, in, out, st);
+      if (p->n1cold)
+        k1_kernel<T, TIO, kFilter><<<(unsigned)p->n1cold, kThreads, p->lds1, st>>>(p->d_cold, p->ncold, in,
+                                                                                  (cx<T>*)p->tbuf);
+      if (p->n2hot)
+        k2_hot_kernel<<<(unsigned)p->n2hot, kThreads, kHotLds, st>>>(p->d_hot, p->nhot, (cx<float>*)p->tbuf,
+                                                                    stage_tab(p, kHotL2));
+      if (p->n2cold)
+        k2_kernel<T, T, kFilter><<<(unsigned)p->n2cold, kThreads, p->lds2, st>>>(p->d_cold, p->ncold,
+                                                                                (cx<T>*)p->tbuf);
+      launch_hot13_all(p, 3, in, out, st);
+      if (p->n1cold)
+        k3_kernel<T, TIO, kFilter><<<(unsigned)p->n1cold, kThreads, p->lds1, st>>>(p->d_cold, p->ncold,
+                                                                                  (const cx<T>*)p->tbuf, out);
+      return;
+    }
+  }
+  k1_kernel<T, TIO, kFilter><<<(unsigned)p->n1, kThreads, p->lds1, st>>>(p->d_segs, p->nseg, in, (cx<T>*)p->tbuf);
+  k2_kernel<T, T, kFilter><<<(unsigned)p->n2, kThreads, p->lds2, st>>>(p->d_segs, p->nseg, (cx<T>*)p->tbuf);
+  k3_kernel<T, TIO, kFilter><<<(unsigned)p->n1, kThreads, p->lds1, st>>>(p->d_segs, p->nseg,
+                                                                         (const cx<T>*)p->tbuf, out);
 }
 
 }  // namespace
@@ -916,16 +1617,15 @@ extern "C" int mk_filt_plan_create_p1(int nseg, const int64_t* desc, int elem_by
   p->nseg = nseg;
   p->borrowed.assign(std::max(1, nseg), 0);
   p->elem_bytes = elem_bytes;
-  const bool hot = getenv("MK_FFT_NO_HOT") == nullptr;
+  const bool hot = elem_bytes == 4 && getenv("MK_FFT_NO_HOT") == nullptr;
   int st = build_segs(nseg, desc, elem_bytes, true, p->h_segs, &p->n1, &p->n2, &p->t_elems, &p->s_elems, &p->lds1,
-                      &p->lds2, hot && elem_bytes == 4, p1, hot);
+                      &p->lds2, hot, p1);
   if (st) { free_filt(p); return st; }
   MK_REQUIRE(p->n1 < INT32_MAX && p->n2 < INT32_MAX, (free_filt(p), MK_ERR_ARG), "too many work items");
-  layout_tables(p);
-  if (hipMalloc((void**)&p->d_hot, std::max<size_t>(1, nseg) * sizeof(Seg)) != hipSuccess ||
-      hipMalloc((void**)&p->d_hotc, std::max<size_t>(1, nseg) * sizeof(Seg)) != hipSuccess ||
+  if (hipMalloc((void**)&p->d_segs, std::max<size_t>(1, nseg) * sizeof(Seg)) != hipSuccess ||
+      hipMalloc((void**)&p->d_hot, std::max<size_t>(1, nseg) * sizeof(Seg)) != hipSuccess ||
       hipMalloc((void**)&p->d_cold, std::max<size_t>(1, nseg) * sizeof(Seg)) != hipSuccess ||
-      hipMalloc(&p->tw, std::max<int64_t>(1, p->tw_all) * 2 * elem_bytes) != hipSuccess) {
+      hipMalloc((void**)&p->d_hot13, std::max<size_t>(1, nseg) * sizeof(Seg)) != hipSuccess) {
     free_filt(p);
     mk::set_error("filter plan: device allocation failed");
     return MK_ERR_ALLOC;
@@ -933,11 +1633,8 @@ extern "C" int mk_filt_plan_create_p1(int nseg, const int64_t* desc, int elem_by
   // spectra are allocated by mk_filt_plan_set_weights: a plan that borrows
   // every segment's spectrum never holds any of its own
   for (auto& sg : p->h_segs) sg.s_ptr = nullptr;
-  if (p->tw_elems) {
-    st = elem_bytes == 4 ? build_tables<float>(p, p->tw, nullptr) : build_tables<double>(p, p->tw, nullptr);
-    if (st == MK_OK) st = elem_bytes == 4 ? build_end_phases<float>(p, nullptr) : build_end_phases<double>(p, nullptr);
-    if (st == MK_OK && hipDeviceSynchronize() != hipSuccess)  // exec may run on another stream
-      st = (mk::set_error("filter plan: twiddle table build failed"), MK_ERR_HIP);
+  if (hot) {
+    st = build_hot_tables(p);
     if (st) { free_filt(p); return st; }
   }
   if (upload(p)) {
@@ -955,7 +1652,7 @@ extern "C" int mk_filt_plan_borrow_spectrum(mk_filt_plan* p, int seg, const mk_f
   MK_REQUIRE(src->have_spec, MK_ERR_ARG, "source plan has no weights");
   Seg& d = p->h_segs[seg];
   const Seg& s = src->h_segs[src_seg];
-  MK_REQUIRE(d.rows == s.rows && d.n == s.n && d.p1 == s.p1 && d.l2 == s.l2 && d.q1 == s.q1, MK_ERR_ARG,
+  MK_REQUIRE(d.rows == s.rows && d.n == s.n && d.p1 == s.p1 && d.l2 == s.l2, MK_ERR_ARG,
              "segment geometry differs (rows %d/%d, n %d/%d)", d.rows, s.rows, d.n, s.n);
   d.s_ptr = s.s_ptr;
   p->borrowed[seg] = 1;
@@ -983,8 +1680,7 @@ extern "C" int mk_filt_plan_info(const mk_filt_plan* p, int64_t* info) {
   return MK_OK;
 }
 
-// Per-segment geometry: out[4*i..] = {P1, P2, cw, P1 P2} of segment i (on the
-// 2^11-row path the length class, see kHotP1).
+// Per-segment FFT geometry: out[4*i..] = {P1, P2, cw, P} of segment i.
 extern "C" int mk_filt_plan_geometry(const mk_filt_plan* p, int64_t* out) {
   MK_REQUIRE(p && out, MK_ERR_ARG, "null pointer");
   for (int i = 0; i < p->nseg; i++) {
@@ -992,7 +1688,7 @@ extern "C" int mk_filt_plan_geometry(const mk_filt_plan* p, int64_t* out) {
     out[4 * i] = s.p1;
     out[4 * i + 1] = int64_t(1) << s.l2;
     out[4 * i + 2] = s.cw;
-    out[4 * i + 3] = (int64_t)s.p1 << s.l2;
+    out[4 * i + 3] = s.t_stride;
   }
   return MK_OK;
 }
@@ -1014,58 +1710,27 @@ extern "C" int mk_filt_plan_set_weights(mk_filt_plan* p, const double* wdct, voi
     if (r) return r;
   }
   // The spectrum is always computed in FP64 (a transient FP64 work buffer)
-  // and stored in the plan's precision, unless FP64 LDS tiles of the general
-  // path would not fit.
+  // and stored in the plan's precision, unless FP64 LDS tiles would not fit.
   size_t l1_64 = 0, l2_64 = 0;
   for (const Seg& sg : p->h_segs) {
-    if (sg.hot) continue;
     Geometry g{sg.l1, sg.l2, sg.cw, sg.p1, (int64_t)sg.p1 << sg.l2};
     l1_64 = std::max(l1_64, lds_k13(g, 8));
     l2_64 = std::max(l2_64, lds_k2(g, 8));
   }
   const bool fp64_pass = l1_64 <= (size_t)kMaxLds && l2_64 <= (size_t)kMaxLds;
   void* tb = nullptr;
-  void* tw64 = nullptr;
-  int r = MK_OK;
-  if (hipMalloc(&tb, std::max<int64_t>(1, p->t_elems) * 16) != hipSuccess ||
-      (p->elem_bytes == 4 && p->tw_elems && hipMalloc(&tw64, p->tw_elems * 16) != hipSuccess)) {
-    if (tb) (void)hipFree(tb);
-    mk::set_error("filter plan: spectrum work allocation (%lld B) failed", (long long)(p->t_elems * 16));
-    return MK_ERR_ALLOC;
+  if (fp64_pass) {
+    MK_HIP(hipMalloc(&tb, std::max<int64_t>(1, p->t_elems) * 16));
+    if (p->elem_bytes == 4) launch_fspec<double, float>(p, wdct, tb, l1_64, l2_64, st);
+    else launch_fspec<double, double>(p, wdct, tb, l1_64, l2_64, st);
+  } else {
+    MK_HIP(hipMalloc(&tb, std::max<int64_t>(1, p->t_elems) * 8));
+    launch_fspec<float, float>(p, wdct, tb, p->lds1, p->lds2, st);
   }
-  if (p->n2hot) {
-    if (p->elem_bytes == 4) {  // the FP64 pass numbers its column tiles differently
-      r = build_tables<double>(p, tw64, st);
-      if (r == MK_OK) r = upload_lists(p, 8);
-    }
-    const cx<double>* tw = (const cx<double>*)(p->elem_bytes == 4 ? tw64 : p->tw);
-    for (int comp = 0; comp < 2 && r == MK_OK; comp++) {
-      launch_hot_fwd<double>(p, kFSpec, wdct, (cx<double>*)tb, tw, comp, st);
-      launch_rows<double>(kFSpec, p->d_hot, p->nhot, p->n2hot, (cx<double>*)tb, tw, comp, p->elem_bytes == 4, st);
-      r = mk::check_launch("filter spectrum");
-    }
-    int64_t rows = 0;
-    for (const Seg& sg : p->h_segs) rows += sg.hot ? sg.rows : 0;
-    if (r == MK_OK) {
-      launch_end_modes(p->d_hot, p->nhot, rows, wdct, p->elem_bytes == 4, st);
-      r = mk::check_launch("end_modes_kernel");
-    }
-  }
-  if (p->n1cold && r == MK_OK) {
-    if (fp64_pass && p->elem_bytes == 4) launch_fspec<double, float>(p, wdct, tb, l1_64, l2_64, st);
-    else if (fp64_pass) launch_fspec<double, double>(p, wdct, tb, l1_64, l2_64, st);
-    else launch_fspec<float, float>(p, wdct, tb, p->lds1, p->lds2, st);
-    r = mk::check_launch("filter spectrum");
-  }
-  if (hipStreamSynchronize(st) != hipSuccess && r == MK_OK)
-    r = (mk::set_error("filter spectrum: stream synchronisation failed"), MK_ERR_HIP);
-  if (p->n2hot && p->elem_bytes == 4) {  // back to the FP32 numbering
-    const int u = upload(p);
-    if (r == MK_OK) r = u;
-  }
-  (void)hipFree(tb);
-  if (tw64) (void)hipFree(tw64);
+  int r = mk::check_launch("filter spectrum");
   if (r == MK_OK) p->have_spec = true;
+  MK_HIP(hipStreamSynchronize(st));
+  MK_HIP(hipFree(tb));
   return r;
 }
 
@@ -1130,91 +1795,24 @@ extern "C" int mk_filt_plan_set_halve(mk_filt_plan* p, int halve_edges) {
 // ---------------------------------------------------------------------------
 // Stand-alone DCT-I (Bluestein), rows of one length n.
 
-namespace {
-// Workspace of the general path (power-of-two P): descriptors, chirp
-// spectrum, rows.
-int64_t dct1_general_bytes(int64_t nrow, int64_t n, int elem_bytes) {
+extern "C" int64_t mk_dct1_workspace_bytes(int64_t nrow, int64_t n, int elem_bytes) {
+  if (n < 2 || nrow < 0 || (elem_bytes != 4 && elem_bytes != 8)) return -1;
   Geometry g = geometry(2 * (n - 1) + 1, elem_bytes);
   return (nrow * g.P + g.P) * 2 * elem_bytes + 4096;
 }
-// Column count of the 2^11-row path for FP64 rows of n points (0: general
-// path), and its workspace: descriptors, chirp spectrum, rows, twiddle
-// tables, chirp.
-int dct1_q1(int64_t n, int elem_bytes) {
-  const int64_t need = 2 * (n - 1) + 1;
-  return elem_bytes == 8 && need > kHotP2 && !getenv("MK_FFT_NO_HOT") ? q1_at_least(need) : 0;
-}
-int64_t dct1_rows_bytes(int64_t nrow, int64_t n, int q) {
-  return ((nrow + 1) * q * kHotP2 + kTwCommon + q1_table_elems(q) + n) * 16 + 4096;
-}
-}  // namespace
-
-extern "C" int64_t mk_dct1_workspace_bytes(int64_t nrow, int64_t n, int elem_bytes) {
-  if (n < 2 || nrow < 0 || (elem_bytes != 4 && elem_bytes != 8)) return -1;
-  const int q = dct1_q1(n, elem_bytes);
-  return q ? dct1_rows_bytes(nrow, n, q) : dct1_general_bytes(nrow, n, elem_bytes);
-}
 
 namespace {
-// FP64 rows through the 2^11-row engine: P = 2^11 q >= 2m+1 points (a
-// power of two on the general path, 1.4 times as many on average), the chirp
-// from a table built once per call.
-int dct1_rows64(const double* x, double* y, int64_t nrow, int64_t n, int q, void* work, hipStream_t st) {
-  unsigned char* w = (unsigned char*)work;
-  const int64_t P = (int64_t)q * kHotP2;
-  cx<double>* V = (cx<double>*)(w + 4096);
-  cx<double>* tb = V + P;
-  cx<double>* tw = tb + nrow * P;
-  cx<double>* qt = tw + kTwCommon;
-  cx<double>* chirp = qt + q1_table_elems(q);
-  Seg s[2] = {};
-  s[0].in_stride = s[0].out_stride = n;
-  s[0].t_stride = P;
-  s[0].s_ptr = V;
-  s[0].tw_off = kTwCommon;
-  s[0].rows = (int32_t)nrow;
-  s[0].n = (int32_t)n;
-  s[0].per2 = (q + 1) / 2;
-  s[0].q1 = q;
-  s[1] = s[0];
-  s[1].rows = 1;
-  const int64_t nb = col_blocks<double>(q);
-  MK_REQUIRE(nrow * nb < INT32_MAX && nrow * s[0].per2 < INT32_MAX, MK_ERR_ARG, "too many rows");
-  Seg* d = (Seg*)w;
-  static_assert(2 * sizeof(Seg) <= 4096, "descriptors");
-  MK_HIP(hipMemcpyAsync(d, s, sizeof(s), hipMemcpyHostToDevice, st));
-  MK_HIP(hipStreamSynchronize(st));
-  launch_col_tables<double>(q, tw, qt, st);
-  launch_chirp(chirp, n, st);
-  const cx<double>* ct = qt + (int64_t)q * kRowTw;
-  launch_cols_fwd<double>(q, kBSpec, d + 1, 1, nb, x, V, tw, ct, chirp, 0, st);
-  launch_rows<double>(kBSpec, d + 1, 1, s[0].per2, V, tw, 0, false, st);
-  launch_cols_fwd<double>(q, kBlue, d, 1, nrow * nb, x, tb, tw, ct, chirp, 0, st);
-  launch_rows<double>(kBlue, d, 1, nrow * s[0].per2, tb, tw, 0, false, st);
-  launch_cols_inv<double>(q, kBlue, d, 1, nrow * nb, tb, y, tw, ct, chirp, st);
-  return mk::check_launch("dct1");
-}
-
 template <typename T, typename TIO>
 int dct1_impl(const TIO* x, TIO* y, int64_t nrow, int64_t n, void* work, int64_t work_bytes, void* stream) {
   MK_REQUIRE(nrow >= 0 && n >= 2, MK_ERR_ARG, "DCT-I needs n >= 2 (got %lld)", (long long)n);
   if (nrow == 0) return MK_OK;
   MK_REQUIRE(x && y && work, MK_ERR_ARG, "null argument");
-  MK_REQUIRE(n < (int64_t(1) << 30) && nrow < INT32_MAX, MK_ERR_ARG, "DCT-I of %lld rows of %lld points is too large",
-             (long long)nrow, (long long)n);
-  // the 2^11-row path wants slightly more than the general one where P is
-  // about the same; a caller's workspace of the general size is still served
-  const int q = dct1_q1(n, sizeof(T));
-  const bool rows = q && work_bytes >= dct1_rows_bytes(nrow, n, q);
-  const int64_t need = dct1_general_bytes(nrow, n, sizeof(T));
-  MK_REQUIRE(rows || work_bytes >= need, MK_ERR_ARG, "workspace too small (%lld < %lld)", (long long)work_bytes,
+  int64_t need = mk_dct1_workspace_bytes(nrow, n, sizeof(T));
+  MK_REQUIRE(work_bytes >= need, MK_ERR_ARG, "workspace too small (%lld < %lld)", (long long)work_bytes,
              (long long)need);
   MK_REQUIRE(((uintptr_t)work & 255) == 0, MK_ERR_ARG, "workspace must be 256-byte aligned");
   allow_lds_all();
   hipStream_t st = mk::as_stream(stream);
-  if constexpr (sizeof(T) == 8) {
-    if (rows) return dct1_rows64(x, y, nrow, n, q, work, st);
-  }
   int64_t desc[6] = {nrow, n, 0, n, 0, n};
   std::vector<Seg> segs;
   int64_t n1, n2, te, se;
@@ -1282,10 +1880,7 @@ extern "C" int mk_dct1_f64_noalloc(const double* x, double* y, int64_t nrow, int
   MK_REQUIRE(nrow >= 0 && n >= 2, MK_ERR_ARG, "DCT-I needs nrow >= 0 and n >= 2 (got %lld, %lld)", (long long)nrow,
              (long long)n);
   if (nrow == 0) return MK_OK;
-  MK_REQUIRE(n < (int64_t(1) << 30), MK_ERR_ARG, "DCT-I of %lld points is too long", (long long)n);
-  const int64_t q = dct1_q1(n, 8);
-  int64_t need = dct1_general_bytes(nrow, n, 8);
-  if (q) need = std::min(need, dct1_rows_bytes(nrow, n, (int)q));
+  const int64_t need = mk_dct1_workspace_bytes(nrow, n, 8);
   MK_REQUIRE(need > 0 && need <= kScratchBytes, MK_ERR_ARG,
              "mk_dct1_f64_noalloc: %lld rows of %lld points need %lld B of workspace, more than its %lld B static "
              "scratch; use mk_dct1_f64 with a caller workspace (or fewer rows per call)",
