@@ -177,13 +177,12 @@ class LevelsNet(_Base):
             self.dims.append(((h + st - 1) // st, (w + st - 1) // st))
         B = self.B
         self.train = train
+        self.c = None
         if train:
-            self.u = [None] + [self._f32(B, 1, h, w) for h, w in self.dims[1:]]  # u[0] is the caller's
-            self.c = [self._f32(B, CH, h, w) for h, w in self.dims]
-            self.gl = [None] + [self._f32(B, 1, h, w) for h, w in self.dims[1:]]  # g[0] is the caller's
+            self._activations()
             self.ql = [None] + [self._f32(B, 1, h, w) for h, w in self.dims[1:]]
             self.cq = self._f32(B, CH, self.H, self.W)
-        else:  # no activations are kept: C_l^T C_l runs as one composed 5x5 stencil per level
+        else:  # precondition() keeps no activations: C_l^T C_l runs as one composed 5x5 stencil per level
             self._steps = (ctypes.c_int32 * self.nlayer)(*self.steps)
             self._tent = int(kind == "tent")
             nb = int(mkgpu.lib.mk_precon_levels_workspace_bytes(self.nlayer, self._steps, B, self.H, self.W))
@@ -195,11 +194,17 @@ class LevelsNet(_Base):
     def workspace_bytes(self):
         return max(int(mkgpu.lib.mk_conv3x3_wgrad_workspace_bytes(self.B, CH, 1, h, w, 1)) for h, w in self.dims)
 
+    def _activations(self):
+        B = self.B
+        self.u = [None] + [self._f32(B, 1, h, w) for h, w in self.dims[1:]]  # u[0] is the caller's
+        self.gl = [None] + [self._f32(B, 1, h, w) for h, w in self.dims[1:]]  # g[0] is the caller's
+        self.c = [self._f32(B, CH, h, w) for h, w in self.dims]
+
     def refresh_adjoint(self):
-        if self.train:
-            return super().refresh_adjoint()
-        mkgpu.check("mk_level_stencils_f32", self.params.data_ptr(), self.nlayer, self.stencils.data_ptr(),
-                    dev.stream_ptr())
+        super().refresh_adjoint()
+        if not self.train:
+            mkgpu.check("mk_level_stencils_f32", self.params.data_ptr(), self.nlayer, self.stencils.data_ptr(),
+                        dev.stream_ptr())
 
     def precondition(self, r, s, z):
         """z = s (alpha s r + K^T K s r) outside training; z overlaps neither."""
@@ -217,7 +222,10 @@ class LevelsNet(_Base):
                     dev.stream_ptr())
 
     def forward(self, u, g0):
-        """g0 = K^T K u, keeping the activations (networks built for training)."""
+        """g0 = K^T K u layer by layer, keeping the activations.  A network built
+        outside training allocates them at its first call."""
+        if self.c is None:
+            self._activations()
         L = self.nlayer
         us = [u] + self.u[1:]
         gs = [g0] + self.gl[1:]

@@ -308,3 +308,25 @@ def test_levels_precon_in_place(env):
     lp.apply_to(rt, z)
     lp.apply_to(rt, rt)
     assert torch.equal(rt, z)
+
+
+@pytest.mark.parametrize("arch,spec", [("levels", (1, 2)), ("tent", (1, 4, 16))])
+def test_levels_forward_outside_training(env, arch, spec):
+    """The layered K^T K u of a network built without training buffers is the
+    training network's, and leaves precondition() as it was."""
+    torch, device, mkgpu = env
+    from minkasi_amd.learned.nets import make_net
+    p, _, r, _, s, _ = _net_and_data(arch, spec, 2, 37, 50)
+    u, out = _t(env, r * s), []
+    for train in (True, False):
+        net = make_net(arch, spec, p, 2, 37, 50, train)
+        net.refresh_adjoint()
+        g = torch.full_like(u, 3.0)
+        net.forward(u, g)
+        out.append(g)
+    assert torch.equal(out[0], out[1])
+    z = [torch.empty_like(u) for _ in range(2)]
+    for zi in z:
+        net.precondition(_t(env, r), _t(env, s), zi)
+        net.forward(u, g)
+    assert torch.equal(z[0], z[1])
