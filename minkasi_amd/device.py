@@ -79,13 +79,18 @@ class HostFetch:
         self.src = t.reshape(-1)
         self.out = np.empty(tuple(t.shape), dtype=dtype)
         on_dev = torch.from_numpy(self.out).dtype
+        size = min(self.kChunk, self.src.numel())
+        # The device buffers come from the caller's stream: torch keeps memory
+        # per stream and hands out 32 side streams in turn, so buffers of the
+        # side streams' own would stay reserved 32 times over, out of reach of
+        # everything else.
+        buffers = [torch.empty(size, dtype=on_dev, device=t.device) for _ in range(2)]
         self.stream = torch.cuda.Stream(device=t.device)
         self.stream.wait_stream(torch.cuda.current_stream(t.device))
-        t.record_stream(self.stream)  # also where result() is never reached
-        size = min(self.kChunk, self.src.numel())
+        for used in (self.src, *buffers):
+            used.record_stream(self.stream)  # also where result() is never reached
         with torch.cuda.stream(self.stream):
-            self.slots = [(torch.empty(size, dtype=on_dev, device=t.device),
-                           torch.empty(size, dtype=on_dev, pin_memory=True), torch.cuda.Event()) for _ in range(2)]
+            self.slots = [(b, torch.empty(size, dtype=on_dev, pin_memory=True), torch.cuda.Event()) for b in buffers]
             for i in range(2):
                 self._issue(i)
 
