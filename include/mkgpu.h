@@ -552,8 +552,8 @@ int mk_adam_f32(float *p, const float *g, float *m, float *v, int32_t n,
  * fit_cm_plus_poly (minkasi/tods/processing.py:510-579) in device pieces.
  * Per column c (sample) of a row-major nrow x ncol block (row stride ld):
  * out[c] = np.median over the rows (the mean of the two middle values for an
- * even count); 1 <= nrow <= 1024.  Replaces np.median(dd, axis=0)
- * (processing.py:568). */
+ * even count, NaN if the column holds one); 1 <= nrow <= 1024.  Replaces
+ * np.median(dd, axis=0) (processing.py:568). */
 int mk_median_cols_f32(const float *dat, int64_t nrow, int64_t ncol,
                        int64_t ld, float *out, void *stream);
 int mk_median_cols_f64(const double *dat, int64_t nrow, int64_t ncol,

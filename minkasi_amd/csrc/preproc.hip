@@ -6,8 +6,9 @@
 //
 //  median_cols   : per sample (column) the median over the detectors (rows),
 //                  numpy semantics (mean of the two middle values for an even
-//                  count), as exact order statistics: one wave per column
-//                  bisects on the values' ordered bit patterns.
+//                  count, NaN if the column holds one), as exact order
+//                  statistics: one wave per column bisects on the values'
+//                  ordered bit patterns.
 //  design        : X[t][k] = P_k(x_t) (k <= ord) and X[t][ord+1+i] =
 //                  P_i(x_t) cm[t] (i < cm_ord), x_t = (t - (n-1)/2) / ((n-1)/2),
 //                  Legendre P by the three-term recurrence, FP64; also X^T.
@@ -98,6 +99,8 @@ __global__ void __launch_bounds__(256) median_cols_kernel(const T* __restrict__ 
       mx = max(mx, in ? x[e] : (K)0);
     }
     K lo = wave_min(mn), hi = ~wave_min((K)~mx);  // x_k is in [lo, hi]
+    // a NaN's key lies above +inf's or below -inf's
+    const bool nan = hi > order_key((T)INFINITY) || lo < order_key((T)-INFINITY);
     int clo = 0, chi = n;                         // keys below lo, keys up to hi
     while (lo < hi && chi - clo > 1) {
       const K mid = lo + (hi - lo) / 2;
@@ -130,7 +133,7 @@ __global__ void __launch_bounds__(256) median_cols_kernel(const T* __restrict__ 
       }
       med = (med + key_value(b)) / T(2);
     }
-    if (lane == 0) out[c0 + c] = med;
+    if (lane == 0) out[c0 + c] = nan ? (T)NAN : med;
   }
 }
 

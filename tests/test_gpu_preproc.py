@@ -130,6 +130,32 @@ def test_median_cols_extreme_values(env, dtype, nrow):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("nrow", [1, 2, 9, 64, 65, 215, 1024])
+def test_median_cols_nan(env, dtype, nrow):
+    """A column with a NaN of either sign and any payload has a NaN median, as
+    np.median gives; its neighbours do not."""
+    torch, device, mkgpu = env
+    rng = np.random.default_rng(nrow)
+    a = rng.standard_normal((nrow, 12)).astype(dtype)
+    u = a.view(np.uint32 if dtype == np.float32 else np.uint64)
+    top = np.finfo(dtype).bits - 1
+    inf = int(np.array(np.inf, dtype=dtype).view(u.dtype))
+    for c, bits in ((1, inf + 1), (3, inf + 1 + (1 << top)), (5, (1 << top) - 1), (7, (2 << top) - 1)):
+        u[rng.integers(nrow), c] = bits
+    a[:, 9] = np.nan
+    a[nrow // 2:, 10] = np.inf
+    a[0, 10] = np.nan
+    at = device.to_device(a)
+    out = torch.empty(12, dtype=at.dtype, device=at.device)
+    print("median nan", dtype.__name__, nrow, flush=True)
+    mkgpu.check("mk_median_cols_" + ("f64" if dtype == np.float64 else "f32"), at.data_ptr(), nrow, 12, 12,
+                out.data_ptr(), device.stream_ptr())
+    got = out.cpu().numpy()
+    assert np.array_equal(got, np.median(a, axis=0), equal_nan=True)
+    assert np.array_equal(np.isnan(got), np.isin(np.arange(12), [1, 3, 5, 7, 9, 10]))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("nrow,n,ncol", [(1, 1, 1), (7, 255, 2), (8, 256, 3), (9, 257, 5), (17, 4096, 6), (5, 4097, 7),
                                          (16, 9001, 8), (3, 300, 11)])
 def test_design_dots_and_apply_edges(env, dtype, nrow, n, ncol):
