@@ -7,8 +7,8 @@
 //  median_cols   : per sample (column) the median over the detectors (rows),
 //                  numpy semantics (mean of the two middle values for an even
 //                  count, NaN if the column holds one), as exact order
-//                  statistics: one wave per column bisects on the values'
-//                  ordered bit patterns.
+//                  statistics of the values' ordered bit patterns: one wave
+//                  per column bisects on them, or sorts up to 64.
 //  design        : X[t][k] = P_k(x_t) (k <= ord) and X[t][ord+1+i] =
 //                  P_i(x_t) cm[t] (i < cm_ord), x_t = (t - (n-1)/2) / ((n-1)/2),
 //                  Legendre P by the three-term recurrence, FP64; also X^T.
@@ -46,6 +46,13 @@ struct KeyOf<float> { using type = uint32_t; };
 template <>
 struct KeyOf<double> { using type = uint64_t; };
 
+// Whether a column whose smallest and largest keys are these holds a NaN: its
+// key lies above +inf's or below -inf's.
+template <typename T>
+__device__ __forceinline__ bool has_nan(typename KeyOf<T>::type lo, typename KeyOf<T>::type hi) {
+  return hi > order_key((T)INFINITY) || lo < order_key((T)-INFINITY);
+}
+
 // Smallest of the wave, in scalar registers.
 __device__ __forceinline__ uint32_t wave_min(uint32_t v) {
 #pragma unroll
@@ -59,6 +66,41 @@ __device__ __forceinline__ uint64_t wave_min(uint64_t v) {
          (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32;
 }
 
+// v of lane l ^ d.  Moves by 1, 2 and 8 stay within a row of 16 lanes and the
+// vector unit makes them; ds_bpermute, which the others take, is what a sort
+// would be bound by.
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v, int d) {
+  if (d == 1) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xb1, 0xf, 0xf, true);   // quad 1 0 3 2
+  if (d == 2) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4e, 0xf, 0xf, true);   // quad 2 3 0 1
+  if (d == 8) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xf, 0xf, true);  // row rotated by 8
+  return (uint32_t)__shfl_xor((int)v, d, 64);
+}
+__device__ __forceinline__ uint64_t lane_xor(uint64_t v, int d) {
+  return (uint64_t)lane_xor((uint32_t)v, d) | (uint64_t)lane_xor((uint32_t)(v >> 32), d) << 32;
+}
+// Lane l's value (l uniform), in scalar registers.
+__device__ __forceinline__ uint32_t lane_value(uint32_t v, int l) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, l);
+}
+__device__ __forceinline__ uint64_t lane_value(uint64_t v, int l) {
+  return (uint64_t)lane_value((uint32_t)v, l) | (uint64_t)lane_value((uint32_t)(v >> 32), l) << 32;
+}
+
+// Bitonic sort of one key per lane, ascending.
+template <typename K>
+__device__ __forceinline__ K wave_sort(K x, int lane) {
+#pragma unroll
+  for (int k = 2; k <= kWave; k <<= 1) {
+#pragma unroll
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      const K y = lane_xor(x, j);
+      const bool low = ((lane & k) == 0) == ((lane & j) == 0);  // this lane takes the smaller one
+      x = (x < y) == low ? x : y;
+    }
+  }
+  return x;
+}
+
 // Bound by the scalar work of the bisection.  A workgroup stages C columns
 // through LDS, so rows are read along their length (a wave per column would
 // fetch a line for every value), and a wave then holds a column in V registers
@@ -68,7 +110,9 @@ __device__ __forceinline__ uint64_t wave_min(uint64_t v) {
 // column takes about log2(nrow) steps more than its values share leading bits,
 // against (6 + log2 V)(7 + log2 V)/2 exchange stages of a full sort.  215 x
 // 100003 FP32: 65 us from 151 us (bitonic sort over lanes and registers, column
-// loads).
+// loads).  Up to 64 rows the 21 stages of a sort, one key a lane, cost less than
+// the bisection's dependent steps: 64 x 100003 21 us FP32 and 31 us FP64, the
+// bisection 42 and 59.
 template <typename T, int V>
 __global__ void __launch_bounds__(256) median_cols_kernel(const T* __restrict__ dat, int64_t nrow, int64_t ncol,
                                                           int64_t ld, int cbits, T* __restrict__ out) {
@@ -88,6 +132,14 @@ __global__ void __launch_bounds__(256) median_cols_kernel(const T* __restrict__ 
   const int ncl = (int)min((int64_t)C, ncol - c0);
   const int k = (n - 1) / 2;  // the lower middle value
   for (int c = threadIdx.x >> 6; c < ncl; c += 4) {
+    if constexpr (V == 1) {
+      const K x = wave_sort(lane < n ? tile[c * pitch + lane] : ~(K)0, lane);  // the padding sorts last
+      const K first = lane_value(x, 0), last = lane_value(x, n - 1);
+      T med = key_value(lane_value(x, k));
+      if (!(n & 1)) med = (med + key_value(lane_value(x, n / 2))) / T(2);
+      if (lane == 0) out[c0 + c] = has_nan<T>(first, last) ? (T)NAN : med;
+      continue;
+    }
     K x[V];
     K mn = ~(K)0, mx = 0;
 #pragma unroll
@@ -99,8 +151,7 @@ __global__ void __launch_bounds__(256) median_cols_kernel(const T* __restrict__ 
       mx = max(mx, in ? x[e] : (K)0);
     }
     K lo = wave_min(mn), hi = ~wave_min((K)~mx);  // x_k is in [lo, hi]
-    // a NaN's key lies above +inf's or below -inf's
-    const bool nan = hi > order_key((T)INFINITY) || lo < order_key((T)-INFINITY);
+    const bool nan = has_nan<T>(lo, hi);
     int clo = 0, chi = n;                         // keys below lo, keys up to hi
     while (lo < hi && chi - clo > 1) {
       const K mid = lo + (hi - lo) / 2;
@@ -274,10 +325,12 @@ int median_cols_impl(const T* dat, int64_t nrow, int64_t ncol, int64_t ld, T* ou
              (long long)ld);
   if (ncol == 0) return MK_OK;
   MK_REQUIRE(dat && out, MK_ERR_ARG, "null pointer");
-  // columns per workgroup: 32 where they fit 20 KB (eight workgroups a CU),
-  // fewer for tall blocks
+  // Columns per workgroup: up to 32, while they fit 20 KB (eight workgroups a
+  // CU) and leave four workgroups a CU; at least one for each wave.
+  // 64 x 4000 FP32 takes 5.8 us with 4 columns a workgroup, 14 with 32; 64 x
+  // 100003 37 us with 4, 30 with 32 (sorted without row moves).
   int cbits = 5;
-  while (cbits > 2 && (((size_t)(nrow | 1) * sizeof(T)) << cbits) > 20 * 1024) cbits--;
+  while (cbits > 2 && ((((size_t)(nrow | 1) * sizeof(T)) << cbits) > 20 * 1024 || (ncol >> cbits) < 1024)) cbits--;
   const size_t lds = ((size_t)(nrow | 1) * sizeof(T)) << cbits;
   const int64_t groups = mk::cdiv(ncol, (int64_t)1 << cbits);
   MK_REQUIRE(groups < INT32_MAX, MK_ERR_ARG, "median: too many columns");

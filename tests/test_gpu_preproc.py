@@ -156,6 +156,24 @@ def test_median_cols_nan(env, dtype, nrow):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("nrow", [3, 63, 64, 65])
+@pytest.mark.parametrize("ncol", [1, 4099, 8191, 8193, 16385, 32769])
+def test_median_cols_column_groups(env, dtype, nrow, ncol):
+    """4 to 32 columns per workgroup with remainders, on both sides of the 64
+    rows that are sorted and not bisected."""
+    torch, device, mkgpu = env
+    a = np.random.default_rng(nrow + ncol).integers(-40, 40, (nrow, ncol + 3)).astype(dtype) / 8  # ties
+    at = device.to_device(a)
+    out = torch.full((ncol + 1,), 9.0, dtype=at.dtype, device=at.device)
+    print("median groups", dtype.__name__, nrow, ncol, flush=True)
+    mkgpu.check("mk_median_cols_" + ("f64" if dtype == np.float64 else "f32"), at.data_ptr(), nrow, ncol, ncol + 3,
+                out.data_ptr(), device.stream_ptr())
+    got = out.cpu().numpy()
+    assert got[ncol] == 9.0
+    assert np.array_equal(got[:ncol], np.median(a[:, :ncol], axis=0))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("nrow,n,ncol", [(1, 1, 1), (7, 255, 2), (8, 256, 3), (9, 257, 5), (17, 4096, 6), (5, 4097, 7),
                                          (16, 9001, 8), (3, 300, 11)])
 def test_design_dots_and_apply_edges(env, dtype, nrow, n, ncol):
