@@ -18,6 +18,7 @@
 //                  the plain product without base).
 #include "common.h"
 
+#include <algorithm>
 #include <cmath>
 
 namespace {
@@ -219,9 +220,19 @@ __global__ void __launch_bounds__(256) design_kernel(const T* __restrict__ cm, i
   }
 }
 
-constexpr int kDotChunk = 4096;  // samples per partial
 constexpr int kMaxCol = 8;
-constexpr int kDotRows = 8;      // rows per workgroup
+constexpr int kDotRows = 8;  // rows per workgroup
+
+// Samples per partial: 4096, down to 512 while two workgroups a CU are not
+// filled.  64 x 50000 FP32: 38 us at 4096, 17 at 512; 215 x 100003: 50 at
+// 4096, 71 at 512.
+constexpr int64_t kDotChunk = 4096, kDotChunkMin = 512, kDotGroups = 512;
+
+int64_t dot_chunk(int64_t n, int64_t nrow) {
+  int64_t chunk = kDotChunk;
+  while (chunk > kDotChunkMin && mk::cdiv(nrow, kDotRows) * mk::cdiv(n, chunk) < kDotGroups) chunk /= 2;
+  return chunk;
+}
 
 // part[(j * nchunk + chunk) * ncol + k] = sum over the chunk of X[t][k] y_j[t].
 // Bandwidth-bound on y: a thread holds one sample's NC design values and
@@ -233,10 +244,10 @@ constexpr int kDotRows = 8;      // rows per workgroup
 template <typename T, int NC>
 __global__ void __launch_bounds__(256) design_dots_kernel(const double* __restrict__ X, int64_t n,
                                                           const T* __restrict__ y, int64_t nrow, int64_t ld,
-                                                          int64_t nchunk, double* __restrict__ part) {
+                                                          int64_t nchunk, int64_t len, double* __restrict__ part) {
   __shared__ double red[4][64];
   const int64_t j0 = (int64_t)blockIdx.y * kDotRows, chunk = blockIdx.x;
-  const int64_t t0 = chunk * kDotChunk, t1 = min(n, t0 + kDotChunk);
+  const int64_t t0 = chunk * len, t1 = min(n, t0 + len);
   const int nr = (int)min((int64_t)kDotRows, nrow - j0);
   double acc[64];
 #pragma unroll
@@ -273,17 +284,19 @@ __global__ void __launch_bounds__(256) design_dots_kernel(const double* __restri
                                                  red[3][threadIdx.x];
 }
 
-// D[k][j] = sum over chunks (in order) of the partials
-__global__ void design_dots_reduce(const double* __restrict__ part, int64_t nrow, int ncol, int64_t nchunk,
-                                   double* __restrict__ D) {
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < nrow * ncol;
-       e += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t j = e / ncol, k = e % ncol;
-    double s = 0.0;
-#pragma unroll 8
-    for (int64_t c = 0; c < nchunk; c++) s += part[(j * nchunk + c) * ncol + k];
-    D[k * nrow + j] = s;
-  }
+// D[k][j] = sum over chunks of the partials, a wave per sum: lane l adds chunks
+// l, l + 64, ... and the lanes' sums are added in a fixed order, so that the
+// many short chunks of a small block do not queue behind one thread's loads.
+__global__ void __launch_bounds__(256) design_dots_reduce(const double* __restrict__ part, int64_t nrow, int ncol,
+                                                          int64_t nchunk, double* __restrict__ D) {
+  const int64_t e = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (e >= nrow * ncol) return;  // whole wave
+  const int64_t j = e / ncol, k = e % ncol;
+  double s = 0.0;
+  for (int64_t c = threadIdx.x & 63; c < nchunk; c += 64) s += part[(j * nchunk + c) * ncol + k];
+#pragma unroll
+  for (int d = 32; d; d >>= 1) s += __shfl_xor(s, d, 64);
+  if ((threadIdx.x & 63) == 0) D[k * nrow + j] = s;
 }
 
 // Bandwidth-bound on base and out: a thread holds one sample's NK design
@@ -359,20 +372,20 @@ int dots_impl(const double* X, int64_t n, int ncol, const T* y, int64_t nrow, in
   MK_REQUIRE(n >= 1 && ncol >= 1 && ncol <= kMaxCol && nrow >= 1 && nrow < 65536 && ld >= n, MK_ERR_ARG,
              "bad design dot sizes");
   MK_REQUIRE(X && y && D && work, MK_ERR_ARG, "null pointer");
-  const int64_t nchunk = mk::cdiv(n, kDotChunk);
+  const int64_t chunk = dot_chunk(n, nrow), nchunk = mk::cdiv(n, chunk);
   MK_REQUIRE(work_bytes >= nrow * nchunk * ncol * 8, MK_ERR_ARG, "workspace too small");
   hipStream_t st = mk::as_stream(stream);
   const dim3 grid((unsigned)nchunk, (unsigned)mk::cdiv(nrow, kDotRows));
   double* part = (double*)work;
   switch (ncol) {
 #define MK_DOTS(NC) \
-  case NC: design_dots_kernel<T, NC><<<grid, 256, 0, st>>>(X, n, y, nrow, ld, nchunk, part); break
+  case NC: design_dots_kernel<T, NC><<<grid, 256, 0, st>>>(X, n, y, nrow, ld, nchunk, chunk, part); break
     MK_DOTS(1); MK_DOTS(2); MK_DOTS(3); MK_DOTS(4); MK_DOTS(5); MK_DOTS(6); MK_DOTS(7); MK_DOTS(8);
 #undef MK_DOTS
   }
   int r = mk::check_launch("design_dots_kernel");
   if (r) return r;
-  design_dots_reduce<<<mk::grid_for(nrow * ncol, 256), 256, 0, st>>>((const double*)work, nrow, ncol, nchunk, D);
+  design_dots_reduce<<<(unsigned)mk::cdiv(nrow * ncol, 4), 256, 0, st>>>((const double*)work, nrow, ncol, nchunk, D);
   return mk::check_launch("design_dots_reduce");
 }
 
@@ -418,7 +431,12 @@ extern "C" int mk_cm_poly_design_f64(const double* cm, int64_t n, int ord, int c
   return design_impl<double>(cm, n, ord, cm_ord, X, Xt, stream);
 }
 extern "C" int64_t mk_design_dots_workspace_bytes(int64_t n, int ncol, int64_t nrow) {
-  return nrow * mk::cdiv(n, kDotChunk) * ncol * 8 + 256;
+  // Never less for a smaller n or nrow, so that the size for the largest call
+  // serves the others: 8 rows of at most 2 kDotGroups shorter chunks.
+  return std::max(nrow * mk::cdiv(n, kDotChunk),
+                  std::min(nrow * mk::cdiv(n, kDotChunkMin), 2 * kDotGroups * kDotRows)) *
+             ncol * 8 +
+         256;
 }
 extern "C" int mk_design_dots_f32(const double* X, int64_t n, int ncol, const float* y, int64_t nrow, int64_t ld,
                                   double* D, void* work, int64_t work_bytes, void* stream) {

@@ -209,3 +209,28 @@ def test_design_dots_and_apply_edges(env, dtype, nrow, n, ncol):
         got = out.cpu().numpy()
         assert np.all(got[:, n:] == 9.0)
         assert np.all(np.abs(got[:, :n] - ref) <= eps * (np.abs(ref) + 20 * np.finfo(np.float64).eps / eps * 100))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("nrow,n,ncol", [(1, 511, 6), (6, 33300, 6), (64, 513, 8), (64, 65537, 3), (130, 40001, 2),
+                                         (520, 33000, 1)])
+def test_design_dots_chunks(env, dtype, nrow, n, ncol):
+    """Chunks of 512, 1024, 2048 and 4096 samples and more of them than a wave
+    has lanes.  A sum passes at most 16 + 6 + 4 + 8 + 6 additions on its way
+    and a product rounds once: 41 eps of the sum of magnitudes."""
+    torch, device, mkgpu = env
+    rng = np.random.default_rng(nrow + n + ncol)
+    X, y = rng.standard_normal((n, ncol)), rng.standard_normal((nrow, n)).astype(dtype)
+    Xt, yt = device.to_device(X), device.to_device(y)
+    nb = int(mkgpu.lib.mk_design_dots_workspace_bytes(n, ncol, nrow))
+    work = torch.empty(nb // 8, dtype=torch.float64, device=yt.device)
+    D = torch.empty((ncol, nrow), dtype=torch.float64, device=yt.device)
+    print("design chunks", dtype.__name__, nrow, n, ncol, flush=True)
+    for _ in range(2):  # the sums repeat bitwise
+        prev = D.clone()
+        mkgpu.check("mk_design_dots_" + ("f64" if dtype == np.float64 else "f32"), Xt.data_ptr(), n, ncol,
+                    yt.data_ptr(), nrow, n, D.data_ptr(), work.data_ptr(), nb, device.stream_ptr())
+    assert torch.equal(prev, D)
+    y64 = y.astype(np.longdouble)
+    ref, mag = X.T.astype(np.longdouble) @ y64.T, np.abs(X.T) @ np.abs(y64.T)
+    assert np.all(np.abs(D.cpu().numpy() - ref) <= 41 * np.finfo(np.float64).eps * mag)
