@@ -639,10 +639,12 @@ __global__ void __launch_bounds__(256) cross_partial_f64(int M, int N, int64_t n
 // Samples per partial: at most 8192 (a partial costs M x N FP64 numbers of
 // workspace), down to 1024 while the tiles alone leave the chip short of two
 // workgroups per CU.  215 x 90001: 1024 gives 880 workgroups, 8192 gave 110.
+constexpr int64_t kCrossChunk = 8192, kCrossChunkMin = 1024, kCrossGroups = 512;
+
 int64_t cross_chunk(int64_t M, int64_t N, int64_t n, bool sym) {
   const int64_t tm = mk::cdiv(M, TB), tiles = sym ? tm * (tm + 1) / 2 : tm * mk::cdiv(N, TB);
-  int64_t chunk = 8192;
-  while (chunk > 1024 && tiles * mk::cdiv(n, chunk) < 512) chunk /= 2;
+  int64_t chunk = kCrossChunk;
+  while (chunk > kCrossChunkMin && tiles * mk::cdiv(n, chunk) < kCrossGroups) chunk /= 2;
   return chunk;
 }
 
@@ -798,13 +800,19 @@ extern "C" int mk_gemm_nn_f64(int64_t M, int64_t N, int64_t K, const double* A, 
 
 namespace {
 int64_t cross_work_bytes(int64_t M, int64_t N, int64_t n, bool sym) {
-  return std::max<int64_t>(1, mk::cdiv(n, cross_chunk(M, N, n, sym))) * M * N * 8 + 256;
+  // Never less for a smaller M, N or n, so that the size for the largest call
+  // serves the others: shorter chunks than kCrossChunk come to less than 2
+  // kCrossGroups tiles in all, of TB x TB numbers (twice that where only half
+  // the tiles are computed).
+  const int64_t most = (sym ? 4 : 2) * kCrossGroups * TB * TB;
+  return std::max(mk::cdiv(n, kCrossChunk) * M * N, std::min(mk::cdiv(n, kCrossChunkMin) * M * N, most)) * 8 + 256;
 }
 
 template <typename T, bool SYM>
 int cross_impl(int64_t M, int64_t N, int64_t n, const T* A, int64_t lda, const T* B, int64_t ldb, double* C,
-               void* work, void* stream) {
-  const int64_t chunk = cross_chunk(M, N, n, SYM), nchunk = std::max<int64_t>(1, mk::cdiv(n, chunk));
+               void* work, int64_t work_bytes, void* stream) {
+  const int64_t chunk = cross_chunk(M, N, n, SYM), nchunk = mk::cdiv(n, chunk);
+  MK_REQUIRE(work_bytes >= nchunk * M * N * 8, MK_ERR_ARG, "workspace too small");
   MK_REQUIRE(nchunk < 65536, MK_ERR_ARG, "n too large");
   dim3 grid((unsigned)mk::cdiv(N, TB), (unsigned)mk::cdiv(M, TB), (unsigned)nchunk);
   hipStream_t st = mk::as_stream(stream);
@@ -821,9 +829,10 @@ extern "C" int64_t mk_gram_workspace_bytes(int64_t M, int64_t n) { return cross_
 extern "C" int mk_gram_f64(int64_t M, int64_t n, const void* D, int d_is_f32, int64_t ldd, double* G, void* work,
                            int64_t work_bytes, void* stream) {
   MK_REQUIRE(M > 0 && n > 0 && D && G && work, MK_ERR_ARG, "bad arguments");
-  MK_REQUIRE(work_bytes >= mk_gram_workspace_bytes(M, n), MK_ERR_ARG, "workspace too small");
-  return d_is_f32 ? cross_impl<float, true>(M, M, n, (const float*)D, ldd, (const float*)D, ldd, G, work, stream)
-                  : cross_impl<double, true>(M, M, n, (const double*)D, ldd, (const double*)D, ldd, G, work, stream);
+  return d_is_f32 ? cross_impl<float, true>(M, M, n, (const float*)D, ldd, (const float*)D, ldd, G, work,
+                                              work_bytes, stream)
+                  : cross_impl<double, true>(M, M, n, (const double*)D, ldd, (const double*)D, ldd, G, work,
+                                              work_bytes, stream);
 }
 
 extern "C" int64_t mk_cross_workspace_bytes(int64_t M, int64_t N, int64_t n) {
@@ -834,8 +843,7 @@ extern "C" int mk_cross_f64(int64_t M, int64_t N, int64_t n, const double* A, in
                             int64_t ldb, double* C, void* work, int64_t work_bytes, void* stream) {
   MK_REQUIRE(M > 0 && N > 0 && n > 0 && A && B && C && work, MK_ERR_ARG, "bad arguments");
   MK_REQUIRE(M < 65536 * TB && N < 65536 * TB && lda >= n && ldb >= n, MK_ERR_ARG, "bad shapes");
-  MK_REQUIRE(work_bytes >= mk_cross_workspace_bytes(M, N, n), MK_ERR_ARG, "workspace too small");
-  return cross_impl<double, false>(M, N, n, A, lda, B, ldb, C, work, stream);
+  return cross_impl<double, false>(M, N, n, A, lda, B, ldb, C, work, work_bytes, stream);
 }
 
 // ---------------------------------------------------------------------------

@@ -84,3 +84,25 @@ def test_smooth_rows_edges(env, n, t_lo, t_hi):
         ref += g[abs(t)] * v
         mag += g[abs(t)] * np.abs(v)
     assert np.all(np.abs(out.cpu().numpy() - ref) <= 1e-12 * mag)  # up to 16385 terms on both sides
+
+
+def test_cross_and_gram_in_a_longer_calls_workspace(env):
+    """511 chunks of 8192 samples are split into shorter ones, 512 are not: the
+    shorter call still runs in the longer one's workspace."""
+    torch, device, mkgpu = env
+    n = 511 * 8192
+    rng = np.random.default_rng(5)
+    A, B = rng.standard_normal((1, n)), rng.standard_normal((2, n))
+    At, Bt = device.to_device(A), device.to_device(B)
+    f64 = dict(dtype=torch.float64, device=At.device)
+    sp = device.stream_ptr()
+    for got, size, call, ref, mag in (
+            (torch.empty((1, 2), **f64), mkgpu.lib.mk_cross_workspace_bytes(1, 2, n + 8192),
+             lambda C, w, nb: mkgpu.check("mk_cross_f64", 1, 2, n, At.data_ptr(), n, Bt.data_ptr(), n, C.data_ptr(),
+                                          w.data_ptr(), nb, sp), A @ B.T, np.abs(A) @ np.abs(B).T),
+            (torch.empty((2, 2), **f64), mkgpu.lib.mk_gram_workspace_bytes(2, n + 8192),
+             lambda C, w, nb: mkgpu.check("mk_gram_f64", 2, n, Bt.data_ptr(), 0, n, C.data_ptr(), w.data_ptr(), nb,
+                                          sp), B @ B.T, np.abs(B) @ np.abs(B).T)):
+        work = torch.empty(int(size) // 8, **f64)
+        call(got, work, int(size))
+        _close(got.cpu().numpy(), ref, mag)
