@@ -17,7 +17,7 @@
 //  a column block of B on one XCD so B is re-read from that XCD's L2.
 //
 //  Setup (once per TOD): the Gram matrix d.d^T and the rotation v.d in
-//  FP64 (plain tiled FMA kernels), feeding the host eigendecomposition that
+//  FP64 (on the FP64 matrix cores), feeding the host eigendecomposition that
 //  stands in for np.linalg.svd's left singular vectors.
 #include "common.h"
 
@@ -475,8 +475,10 @@ __global__ void split_matrix_kernel(const double* __restrict__ a, int64_t M, int
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 constexpr int TK = 16;
 
+template <typename T, int W = 4>
+struct alignas(sizeof(T)) Row { T v[W]; };  // consecutive elements at element alignment
 template <typename T>
-struct alignas(sizeof(T)) Row4 { T v[4]; };  // four elements at element alignment
+struct Vec4 { typedef T type __attribute__((ext_vector_type(4))); };
 
 __device__ __forceinline__ f64x4 mfma_f64(double a, double b, f64x4 c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
@@ -487,7 +489,7 @@ template <typename T>
 __device__ __forceinline__ f64x4 load4(const T* __restrict__ p, int64_t left) {
   f64x4 r;
   if (left >= 4) {
-    const Row4<T> q = *reinterpret_cast<const Row4<T>*>(p);
+    const Row<T> q = *reinterpret_cast<const Row<T>*>(p);
 #pragma unroll
     for (int e = 0; e < 4; e++) r[e] = (double)q.v[e];
   } else {
@@ -497,16 +499,34 @@ __device__ __forceinline__ f64x4 load4(const T* __restrict__ p, int64_t left) {
   return r;
 }
 
+// Four elements of a row as they are, W at a time and 16 W apart, 0 from left on.
+template <int W, typename T>
+__device__ __forceinline__ typename Vec4<T>::type load_row(const T* __restrict__ p, int left) {
+  typename Vec4<T>::type r;
+#pragma unroll
+  for (int h = 0; h < 4 / W; h++, p += 16 * W, left -= 16 * W) {
+    if (left >= W) {
+      const Row<T, W> q = *reinterpret_cast<const Row<T, W>*>(p);
+#pragma unroll
+      for (int e = 0; e < W; e++) r[W * h + e] = q.v[e];
+    } else {
+#pragma unroll
+      for (int e = 0; e < W; e++) r[W * h + e] = e < left ? p[e] : T(0);
+    }
+  }
+  return r;
+}
+
 // C[M x N] = A[M x K] . B[K x N]; A FP64 row-major (lda), B of type TBT (ldb),
 // C FP64 (ldc).  Bound by the matrix cores, whose FP64 rate is the vector
 // unit's, but which take their operands once per 16 products: a wave owns 32 x
 // 64 of C and reads both operands from memory into the fragments (B in rows of
-// 64 columns, lane l the columns 4 (l % 16) + j of tile j; A is small and stays
-// in the caches), loading a step ahead.  rw of the workgroup's 4 waves go down
-// the rows, so that they share B's lines.  215 x 215 x 90001, B FP32: 308 us
-// from 375 (64 x 64 tiles through LDS on the vector unit); 64 x 64 x 65536,
-// FP64: 24 us from 34.
-template <typename TBT>
+// 64 columns, of which a lane takes W consecutive ones at a time; A is small
+// and stays in the caches), loading a step ahead.  rw of the workgroup's 4 waves
+// go down the rows, so that they share B's lines.  215 x 215 x 90001, B FP32:
+// 201 us (288 with the conversion beside the load, 328 with 64 x 64 tiles
+// through LDS on the vector unit); 64 x 64 x 65536, FP64: 24 us from 30.
+template <typename TBT, int W>
 __global__ void __launch_bounds__(256) gemm_nn_f64(int M, int N, int K, const double* __restrict__ A, int64_t lda,
                                                    const TBT* __restrict__ B, int64_t ldb, double* __restrict__ C,
                                                    int64_t ldc, int rw) {
@@ -516,7 +536,7 @@ __global__ void __launch_bounds__(256) gemm_nn_f64(int M, int N, int K, const do
   const int lr = lane & 15, lk = 4 * (lane >> 4);
   const double* a0 = A + (int64_t)min(m0 + lr, M - 1) * lda + lk;       // rows past M repeat the last one
   const double* a1 = A + (int64_t)min(m0 + 16 + lr, M - 1) * lda + lk;  // and are not stored
-  const int nc = n0 + 4 * lr;
+  const int nc = n0 + W * lr;
   const TBT* b0 = B + nc;
   const int nleft = N - nc;  // columns from this lane's first one
   f64x4 acc[2][4];
@@ -524,16 +544,20 @@ __global__ void __launch_bounds__(256) gemm_nn_f64(int M, int N, int K, const do
   for (int i = 0; i < 2; i++)
 #pragma unroll
     for (int j = 0; j < 4; j++) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
-  auto load = [&](int k0, f64x4& x0, f64x4& x1, f64x4 (&y)[4]) {
+  // B is converted where it is used: a conversion beside its load would wait
+  // for it
+  using Raw = typename Vec4<TBT>::type;
+  auto load = [&](int k0, f64x4& x0, f64x4& x1, Raw (&y)[4]) {
     x0 = load4(a0 + k0, K - k0 - lk);
     x1 = load4(a1 + k0, K - k0 - lk);
 #pragma unroll
     for (int c = 0; c < 4; c++) {
       const int k = k0 + lk + c;
-      y[c] = load4(b0 + (int64_t)min(k, K - 1) * ldb, k < K ? nleft : 0);
+      y[c] = load_row<W>(b0 + (int64_t)min(k, K - 1) * ldb, k < K ? nleft : 0);
     }
   };
-  f64x4 x0, x1, y[4], p0, p1, q[4];
+  f64x4 x0, x1, p0, p1;
+  Raw y[4], q[4];
   load(0, x0, x1, y);
   for (int k0 = 0; k0 < K; k0 += TK) {
     const bool more = k0 + TK < K;
@@ -542,8 +566,8 @@ __global__ void __launch_bounds__(256) gemm_nn_f64(int M, int N, int K, const do
     for (int c = 0; c < 4; c++)
 #pragma unroll
       for (int j = 0; j < 4; j++) {
-        acc[0][j] = mfma_f64(x0[c], y[c][j], acc[0][j]);
-        acc[1][j] = mfma_f64(x1[c], y[c][j], acc[1][j]);
+        acc[0][j] = mfma_f64(x0[c], (double)y[c][j], acc[0][j]);
+        acc[1][j] = mfma_f64(x1[c], (double)y[c][j], acc[1][j]);
       }
     if (more) {
       x0 = p0;
@@ -559,12 +583,19 @@ __global__ void __launch_bounds__(256) gemm_nn_f64(int M, int N, int K, const do
       const int gm = m0 + 16 * i + 4 * r + (lane >> 4);
       if (gm >= M) continue;
       double* out = C + (int64_t)gm * ldc + nc;
-      if (nleft >= 4) {
-        *reinterpret_cast<Row4<double>*>(out) = {acc[i][0][r], acc[i][1][r], acc[i][2][r], acc[i][3][r]};
-      } else {
 #pragma unroll
-        for (int j = 0; j < 4; j++)
-          if (j < nleft) out[j] = acc[i][j][r];
+      for (int h = 0; h < 4 / W; h++) {
+        const int left = nleft - 16 * W * h;
+        if (left >= W) {
+          Row<double, W> v;
+#pragma unroll
+          for (int e = 0; e < W; e++) v.v[e] = acc[i][W * h + e][r];
+          *reinterpret_cast<Row<double, W>*>(out + 16 * W * h) = v;
+        } else {
+#pragma unroll
+          for (int e = 0; e < W; e++)
+            if (e < left) out[16 * W * h + e] = acc[i][W * h + e][r];
+        }
       }
     }
 }
@@ -791,10 +822,15 @@ extern "C" int mk_gemm_nn_f64(int64_t M, int64_t N, int64_t K, const double* A, 
   const int rw = M <= 32 ? 1 : M <= 64 ? 2 : 4;  // waves down the rows
   dim3 grid((unsigned)mk::cdiv(N, 64 * (4 / rw)), (unsigned)mk::cdiv(M, 32 * rw));
   hipStream_t st = mk::as_stream(stream);
-  if (b_is_f32)
-    gemm_nn_f64<float><<<grid, 256, 0, st>>>((int)M, (int)N, (int)K, A, lda, (const float*)B, ldb, C, ldc, rw);
-  else
-    gemm_nn_f64<double><<<grid, 256, 0, st>>>((int)M, (int)N, (int)K, A, lda, (const double*)B, ldb, C, ldc, rw);
+  auto launch = [&](auto kernel, auto b) {
+    kernel<<<grid, 256, 0, st>>>((int)M, (int)N, (int)K, A, lda, b, ldb, C, ldc, rw);
+  };
+  // Up to two steps of K the stores bound the call, and pairs of columns make
+  // them contiguous over 16 lanes: 512 x 8 x 50001 FP64 42 us, 50 with fours;
+  // 512 x 64 x 50001 97 and 93.
+  const bool thin = K <= 2 * TK;
+  if (b_is_f32) launch(thin ? gemm_nn_f64<float, 2> : gemm_nn_f64<float, 4>, (const float*)B);
+  else launch(thin ? gemm_nn_f64<double, 2> : gemm_nn_f64<double, 4>, (const double*)B);
   return mk::check_launch("gemm_nn_f64");
 }
 

@@ -38,6 +38,27 @@ def test_gemm_nn_edges(env, dtype, M, K, N):
     _close(got[:, :N], a @ b, np.abs(a) @ np.abs(b))
 
 
+@pytest.mark.parametrize("K", [1, 16, 17, 32, 33])
+@pytest.mark.parametrize("N", [1, 2, 3, 31, 33, 62, 63, 66, 67, 97, 125])
+def test_gemm_nn_column_groups(env, K, N):
+    """Pairs (K up to 32) and fours of columns per lane, at every remainder."""
+    torch, device, mkgpu = env
+    M, ldc = 37, N + 1
+    rng = np.random.default_rng(K + 100 * N)
+    A = rng.standard_normal((M, K))
+    At = device.to_device(A)
+    print("gemm groups", K, N, flush=True)
+    for dtype in (np.float32, np.float64):
+        B = rng.standard_normal((K, N)).astype(dtype)
+        Bt = device.to_device(B)
+        C = torch.full((M, ldc), 9.0, dtype=torch.float64, device=At.device)
+        mkgpu.check("mk_gemm_nn_f64", M, N, K, At.data_ptr(), K, Bt.data_ptr(), int(dtype == np.float32), N,
+                    C.data_ptr(), ldc, device.stream_ptr())
+        b, got = B.astype(np.float64), C.cpu().numpy()
+        assert np.all(got[:, N:] == 9.0)
+        _close(got[:, :N], A @ b, np.abs(A) @ np.abs(b))
+
+
 @pytest.mark.parametrize("M,N,n", [(1, 1, 1), (16, 17, 15), (31, 33, 16), (64, 65, 1025), (65, 3, 2049), (130, 70, 5003)])
 def test_cross_and_gram_edges(env, M, N, n):
     torch, device, mkgpu = env
