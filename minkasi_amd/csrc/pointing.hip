@@ -133,16 +133,24 @@ __global__ void __launch_bounds__(256) raster_kernel(const double* __restrict__ 
                                                      const double* __restrict__ dra, const double* __restrict__ ddec,
                                                      int64_t ndet, int64_t ndata, CarWcs w, int32_t nx, int32_t ny,
                                                      int32_t* __restrict__ ipix, int64_t* nbad) {
-  // 256 samples of one detector at a time: the division is the workgroup's,
-  // not every sample's
-  const int64_t nt = (ndata + 255) / 256;
-  for (int64_t b = blockIdx.x; b < ndet * nt; b += gridDim.x) {
-    const int64_t d = b / nt, t = (b - d * nt) * 256 + threadIdx.x;
+  // 64 consecutive samples of the block a wave: the division is the wave's, not
+  // every sample's, and rows of any length fill the lanes (1000 detectors of 20
+  // samples: 6.4 us, 25.6 with 256 samples of one detector a workgroup; 215 x
+  // 100003: 291 us, 373 with a division per sample and the looping remainders)
+  const int64_t n = ndet * ndata;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  for (int64_t base = ((int64_t)blockIdx.x * 4 + wave) * 64; base < n; base += (int64_t)gridDim.x * 256) {
+    int64_t d = base / ndata, t = base - d * ndata + lane;
+    if (t >= ndata) {  // past the first detector's end: into the next, or beyond it in rows shorter than a wave
+      const int64_t q = ndata >= 64 ? 1 : (uint32_t)t / (uint32_t)ndata;
+      d += q;
+      t -= q * ndata;
+    }
     bool bad = false;
-    if (t < ndata) {
+    if (base + lane < n) {
       double px, py;
       car_one(ra_b[t] + dra[d], dec_b[t] + ddec[d], w, &px, &py);
-      ipix[d * ndata + t] = to_ipix(px, py, nx, ny, &bad);
+      ipix[base + lane] = to_ipix(px, py, nx, ny, &bad);
     }
     count_bad(bad, nbad);
   }

@@ -92,6 +92,30 @@ def test_pix_raster_variant_equals_full(env):
     assert np.array_equal(ip.cpu().numpy(), ip_full)
 
 
+@pytest.mark.parametrize("ndet,n", [(1, 1), (300, 1), (7, 2), (65, 20), (3, 63), (5, 64), (5, 65), (9, 127), (4, 255),
+                                    (3, 256), (3, 257), (2, 40003)])
+def test_pix_raster_row_lengths(env, ndet, n):
+    """Rows shorter and longer than a wave, and remainders of both, against the
+    same pointing written out; some samples are out of the map."""
+    torch, device, mkgpu = env
+    rng = np.random.default_rng(ndet + n)
+    from minkasi_amd.maps.wcs import CarWCS
+    prm = CarWCS((180.0, 60.0), (-2 / 3600, 2 / 3600), (65, 50)).params10()
+    ra_b, dec_b = np.pi + rng.uniform(-1, 1, n) * 300 * ARCSEC, np.deg2rad(60) + rng.uniform(-1, 1, n) * 100 * ARCSEC
+    dra, ddec = rng.uniform(-1, 1, ndet) * 20 * ARCSEC, rng.uniform(-1, 1, ndet) * 20 * ARCSEC
+    t = [device.to_device(a, torch.float64) for a in (ra_b, dec_b, dra, ddec)]
+    full = [(t[0] + t[2][:, None]).contiguous(), (t[1] + t[3][:, None]).contiguous()]
+    ip = torch.full((2, ndet * n + 1), -7, dtype=torch.int32, device=t[0].device)
+    nbad = torch.zeros(2, dtype=torch.int64, device=t[0].device)
+    print("raster", ndet, n, flush=True)
+    mkgpu.check("mk_pix_from_raster_car", *(a.data_ptr() for a in t), ndet, n, prm.ctypes.data, 130, 100,
+                ip[0].data_ptr(), nbad[0:].data_ptr(), device.stream_ptr())
+    mkgpu.check("mk_pix_from_radec_car", full[0].data_ptr(), full[1].data_ptr(), ndet * n, prm.ctypes.data, 130, 100,
+                ip[1].data_ptr(), nbad[1:].data_ptr(), device.stream_ptr())
+    assert torch.equal(ip[0], ip[1]) and nbad[0] == nbad[1]
+    assert ip[0, -1] == -7
+
+
 def test_pix_counts_out_of_range(env):
     rng = np.random.default_rng(13)
     ra_b, dec_b, dra, ddec = raster_pointing(rng, 4, 2000)
