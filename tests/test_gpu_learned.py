@@ -320,11 +320,14 @@ def test_levels_forward_outside_training(env, arch, spec):
     u, out = _t(env, r * s), []
     for train in (True, False):
         net = make_net(arch, spec, p, 2, 37, 50, train)
-        net.refresh_adjoint()
-        g = torch.full_like(u, 3.0)
-        net.forward(u, g)
-        out.append(g)
-    assert torch.equal(out[0], out[1])
+        for scale in (1.0, -0.5):  # new weights reach the adjoint layers too
+            net.params.mul_(scale)
+            net.refresh_adjoint()
+            g = torch.full_like(u, 3.0)
+            net.forward(u, g)
+            out.append(g)
+    assert torch.equal(out[0], out[2]) and torch.equal(out[1], out[3])
+    assert not torch.equal(out[0], out[1])
     z = [torch.empty_like(u) for _ in range(2)]
     for zi in z:
         net.precondition(_t(env, r), _t(env, s), zi)
