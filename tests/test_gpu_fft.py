@@ -240,3 +240,62 @@ def test_filter_fp32_longer_column_lengths_are_exact(env):
         p = np.asarray([bad], dtype=np.int32)
         with pytest.raises(mkgpu.MkError):
             mkgpu.check("mk_filt_plan_create_p1", 1, desc.ctypes.data, 4, p.ctypes.data, ctypes.byref(h))
+
+
+def _noise_weights(x, fwhm=50.0):
+    """The noise model's weights: the inverse of the power spectrum smoothed by
+    a Gaussian, 0 for the constant."""
+    n = x.shape[-1]
+    g = np.exp(-0.5 * (np.arange(n) / (fwhm / np.sqrt(8 * np.log(2)))) ** 2)
+    g /= g[0] + g[-1] + 2 * g[1:-1].sum()
+    p = sf.dct(x, type=1) ** 2
+    w = 1 / (sf.dct(sf.dct(p, type=1) * sf.dct(g, type=1), type=1) / (2 * (n - 1)))
+    w[:, 0] = 0
+    return w
+
+
+@pytest.mark.parametrize("kind", ["white", "mildly red", "common mode"])
+@pytest.mark.parametrize("n", [21845, 21846, 87381, 87382, 90001])
+def test_filter_fp32_error_by_band(env, kind, n):
+    """The error lies where rounding puts it, band by band of cosine modes: on
+    rows whose low modes are far above the rest (and whose weights are far
+    below), a norm-wise bound sees the high modes alone.  Rounding adds u =
+    2^-24 of the row's rms mode, times the band's weight, on the way in and u
+    of the result's rms mode on the way out, times about 0.6 sqrt(log2 of the
+    transform's length) = 2.5 each; 8 leaves room for bands of three modes.
+    The lengths just fit and just miss a column count."""
+    torch, device, mkgpu = env
+    rng = np.random.default_rng(n)
+    x = 0.1 * rng.standard_normal((4, n))
+    walk = np.cumsum(rng.standard_normal((4, n)), axis=1)
+    if kind == "mildly red":
+        x += 1e-4 * walk
+    elif kind == "common mode":
+        x = x / 8 + 0.05 * walk
+    x = x.astype(np.float32).astype(np.float64)
+    w = _noise_weights(x)
+    desc = np.asarray([4, n, 0, n, 0, n], dtype=np.int64)
+    h = ctypes.c_void_p()
+    mkgpu.check("mk_filt_plan_create", 1, desc.ctypes.data, 4, ctypes.byref(h))
+    try:
+        wdt = device.to_device(sf.dct(w, type=1))
+        mkgpu.check("mk_filt_plan_set_weights", h, wdt.data_ptr(), device.stream_ptr())
+        mkgpu.check("mk_filt_plan_set_halve", h, 0)
+        xt = device.to_device(x.astype(np.float32))
+        yt = torch.empty_like(xt)
+        print("filter bands", kind, n, flush=True)
+        mkgpu.check("mk_filt_plan_exec_f32", h, xt.data_ptr(), yt.data_ptr(), device.stream_ptr())
+        out = yt.cpu().numpy().astype(np.float64)
+    finally:
+        mkgpu.check("mk_filt_plan_destroy", h)
+    X = sf.dct(x, type=1)
+    err = sf.dct(out - sf.dct(X * w, type=1), type=1)
+    scale = 2 * (n - 1)  # the DCT-I pair's
+
+    def rms(a):
+        return np.sqrt((a ** 2).mean(axis=1))
+
+    for a, b in ((2, 5), (5, 20), (20, 100), (100, 1000), (1000, n)):
+        bound = 2.0 ** -24 * scale * (rms(w[:, a:b]) * rms(X) + rms(X * w))
+        got = np.sqrt(((rms(err[:, a:b]) / bound) ** 2).mean())
+        assert got < 8, (a, b, got)

@@ -116,6 +116,25 @@ def test_pix_raster_row_lengths(env, ndet, n):
     assert ip[0, -1] == -7
 
 
+@pytest.mark.parametrize("lat0", [60.0, 30.0])
+def test_pix_exact_angles(env, lat0):
+    """Pointing at exact multiples of 90 and 180 degrees from the pole's
+    longitude, at the equator and the poles, where the rotation takes sine and
+    cosine exactly and the latitude directly, and just beside them, against the
+    host oracle.  The math libraries differ by a few roundings, some 1e-12 of
+    the 324000 pixels that 180 degrees span."""
+    w = dict(crval=np.array([180.0, lat0]), cdelt=np.array([-2 / 3600, 2 / 3600]), crpix=np.array([1.0, 1.0]))
+    deg = np.array([0.0, 90.0, 180.0, 270.0, 360.0, 450.0, -90.0, -180.0, 720.0, 1e-9, 89.999999999, 179.9999999, 33.0])
+    ra, dec = (a.ravel() * np.pi / 180 for a in np.meshgrid(deg, [0.0, 90.0, -90.0, 45.0, 1e-10, 89.9999999]))
+    assert np.sum(np.fmod(ra * 180 / np.pi - core.car_euler(w)[0], 90.0) == 0.0) == 54
+    _, _, px, py = _gpu_pix(env, w, 1 << 14, 1 << 14, ra, dec)
+    qx, qy = core.car_world2pix(w, ra, dec)
+    tol, turn = 1e-12 * 324000, 648000  # +-180 degrees are one longitude
+    dx = np.abs(px - qx)
+    assert np.all(np.minimum(dx, np.abs(dx - turn)) < tol)
+    assert np.all(np.abs(py - qy) < tol)
+
+
 def test_pix_counts_out_of_range(env):
     rng = np.random.default_rng(13)
     ra_b, dec_b, dra, ddec = raster_pointing(rng, 4, 2000)
