@@ -433,7 +433,9 @@ int mk_defl_plan_destroy(mk_defl_plan *plan);
 /* FP64 setup GEMMs (NoiseSmoothedSVD.__init__, noise.py:650 and :667):
  * C = A.B (A FP64; B FP32 if b_is_f32 else FP64), and the Gram matrix
  * G = D.D^T (M x M) that replaces the SVD's left singular vectors
- * (eigenvectors of D.D^T).  work: mk_gram_workspace_bytes(M, n) bytes. */
+ * (eigenvectors of D.D^T).  work: mk_gram_workspace_bytes(M, n) bytes; the
+ * size for the largest call serves smaller ones, here and for mk_cross_f64
+ * and mk_design_dots_*. */
 int mk_gemm_nn_f64(int64_t M, int64_t N, int64_t K, const double *A,
                    int64_t lda, const void *B, int b_is_f32, int64_t ldb,
                    double *C, int64_t ldc, void *stream);
