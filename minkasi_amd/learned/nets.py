@@ -183,7 +183,6 @@ class LevelsNet(_Base):
             self.ql = [None] + [self._f32(B, 1, h, w) for h, w in self.dims[1:]]
             self.cq = self._f32(B, CH, self.H, self.W)
         else:  # precondition() keeps no activations: C_l^T C_l runs as one composed 5x5 stencil per level
-            self._wt_stale = True
             self._steps = (ctypes.c_int32 * self.nlayer)(*self.steps)
             self._tent = int(kind == "tent")
             nb = int(mkgpu.lib.mk_precon_levels_workspace_bytes(self.nlayer, self._steps, B, self.H, self.W))
@@ -202,11 +201,11 @@ class LevelsNet(_Base):
         self.c = [self._f32(B, CH, h, w) for h, w in self.dims]
 
     def refresh_adjoint(self):
-        if self.train:
-            return super().refresh_adjoint()
-        self._wt_stale = True  # the adjoint weights are forward()'s alone
-        mkgpu.check("mk_level_stencils_f32", self.params.data_ptr(), self.nlayer, self.stencils.data_ptr(),
-                    dev.stream_ptr())
+        if self.c is not None:  # the adjoint weights are forward()'s alone
+            super().refresh_adjoint()
+        if not self.train:
+            mkgpu.check("mk_level_stencils_f32", self.params.data_ptr(), self.nlayer, self.stencils.data_ptr(),
+                        dev.stream_ptr())
 
     def precondition(self, r, s, z):
         """z = s (alpha s r + K^T K s r) outside training; z overlaps neither."""
@@ -225,12 +224,11 @@ class LevelsNet(_Base):
 
     def forward(self, u, g0):
         """g0 = K^T K u layer by layer, keeping the activations.  A network built
-        outside training allocates them at its first call."""
+        outside training allocates them, and makes the adjoint weights that
+        refresh_adjoint() keeps up from then on, at its first call."""
         if self.c is None:
             self._activations()
-        if not self.train and self._wt_stale:
             super().refresh_adjoint()
-            self._wt_stale = False
         L = self.nlayer
         us = [u] + self.u[1:]
         gs = [g0] + self.gl[1:]

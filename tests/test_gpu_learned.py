@@ -333,3 +333,28 @@ def test_levels_forward_outside_training(env, arch, spec):
         net.precondition(_t(env, r), _t(env, s), zi)
         net.forward(u, g)
     assert torch.equal(z[0], z[1])
+
+
+def test_levels_forward_replayed_with_new_weights(env):
+    """A captured forward() outside training reads the weights of the last
+    refresh_adjoint() at every replay."""
+    torch, device, mkgpu = env
+    from minkasi_amd.learned.nets import make_net
+    p, _, r, _, s, _ = _net_and_data("tent", (1, 4), 1, 37, 50)
+    net = make_net("tent", (1, 4), p, 1, 37, 50)
+    net.refresh_adjoint()
+    u = _t(env, r * s)
+    g, want = torch.empty_like(u), torch.empty_like(u)
+    net.forward(u, g)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        net.forward(u, g)
+    for scale in (1.0, -0.5, 3.0):
+        net.params.mul_(scale)
+        net.refresh_adjoint()
+        graph.replay()
+        torch.cuda.synchronize()
+        got = g.clone()
+        net.forward(u, want)
+        assert torch.equal(got, want)
